@@ -321,7 +321,8 @@ int pl_lora_fused_stacked(int32_t dtype, const void* x, int64_t ldx, int32_t K, 
 /* Row-based LoRA on the slot arena for shapes the tiled path rejects
  * (any K, N, strides, alignment).  Writes y[b*row_len+m] for m < seq_len[b].
  * Rows whose slot is <= 0 or >= num_slots get no LoRA.  tmp is
- * [rows*row_len][ldt] fp32 scratch with ldt >= the largest rank. */
+ * [rows*row_len][ldt] fp32 scratch with ldt >= the largest rank (written
+ * for ldt above 256 only: up to there the intermediate stays on chip). */
 int pl_lora_apply_rows(int32_t dtype, const void* x, int64_t ldx, int32_t K, void* y,
                        int64_t ldy, int32_t N, const void* arena, const pl_slot_entry* table,
                        int32_t num_slots, int32_t num_modules, int32_t module,

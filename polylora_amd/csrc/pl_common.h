@@ -187,6 +187,18 @@ int pl_fused_phase(int mode, int32_t dtype, const void* x, int64_t ldx, int32_t 
                    int64_t group_cap, int32_t group_tokens, int32_t slices, int32_t epilogue,
                    void* stream);
 
+// The LoRA of rows straight from the row -> slot map and lengths, at any K, N,
+// stride and element alignment (sgmv_wide.hip), for rank capacities up to
+// kWideRankMax.  Returns PL_WIDE_DECLINED, having launched nothing, for what
+// it does not take.
+constexpr int kWideRankMax = 256;
+constexpr int PL_WIDE_DECLINED = -101;
+int pl_wide_rows_launch(int32_t dtype, const void* x, int64_t ldx, int32_t K, void* y, int64_t ldy,
+                        int32_t N, const void* arena, const pl_slot_entry* table, int32_t num_slots,
+                        int32_t num_modules, int32_t module, const int32_t* row_slot,
+                        const int32_t* seq_lens, int32_t rows, int32_t row_len, int32_t rank_cap,
+                        int32_t epilogue, void* stream);
+
 // MFMA path of the reference-layout operator API (sgmv_refop.hip).  Both
 // return PL_REFOP_DECLINED, having launched nothing, when there is neither a
 // workspace nor parts, or the shape is not one the tiled kernels take; the

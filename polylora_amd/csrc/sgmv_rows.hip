@@ -3,10 +3,10 @@
 // They serve two callers: the reference-layout operator API
 // (sgmv_lora_a_fwd / sgmv_lora_b_fwd, sgmv.py:141-175 and :278-328, weights
 // [slots][k][n] with arbitrary strides) where its MFMA path (sgmv_refop.hip)
-// declines the shape or gets no workspace, and MultiLoraLinear shapes the
-// tiled kernels reject (K or N not a multiple of the 16-byte chunk,
-// unaligned rows).  Throughput is not their goal; the tiled kernels carry
-// the hot path.
+// declines the shape or gets no workspace, and, on the slot arena, rank
+// capacities above kWideRankMax (every other row call of the slot arena runs
+// the MFMA kernel of sgmv_wide.hip: 5 to 80 times as fast at 1 to 4096 rows).
+// Throughput is not their goal.
 //
 // Shrink: one wave per token row; lanes stride K, each rank column is a
 // wave-wide dot product finished with a butterfly reduction.
@@ -351,6 +351,10 @@ extern "C" int pl_lora_apply_rows(int32_t dtype, const void* x, int64_t ldx, int
     pl_set_error("pl_lora_apply_rows: null pointer");
     return PL_ERR_ARG;
   }
+  const int wide = pl_wide_rows_launch(dtype, x, ldx, K, y, ldy, N, arena, table, num_slots,
+                                       num_modules, module, row_slot, seq_lens, rows, row_len, ldt,
+                                       epilogue, stream);
+  if (wide != PL_WIDE_DECLINED) return wide;
   const int32_t nblk = (N + 255) / 256;
   if (!pl_grid_fits(T * nblk, 256)) {
     pl_set_error("pl_lora_apply_rows: grid too large");

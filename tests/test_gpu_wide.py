@@ -1,0 +1,75 @@
+"""The wide-workgroup row kernel (lora_apply_rows) at the edges of its tiles, against the oracle.
+
+K and N around a chunk, a wave load and a 16-wave column step; ranks around a
+pass and past one; rows around a 16-position tile, some empty, some on the base
+adapter; x and y with odd row strides from an odd element, so no access is
+16-byte aligned.  Rank capacities above 256 take the plain row kernels.
+
+Reference: the fallback of layers.py:112-134 (reference_forward).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle.lora import reference_forward
+from polylora_amd import sgmv
+from tests._util import make_cache, oracle_slot_tensors, peft_layer, tol_for
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # rows, row_len, K, N, ranks
+    (3, 1, 1, 1, [1, 2]),
+    (5, 15, 7, 9, [3, 16]),
+    (4, 16, 31, 63, [15, 16]),
+    (4, 17, 33, 65, [17, 32]),
+    (6, 33, 520, 513, [16, 33]),
+    (2, 40, 1025, 1023, [4, 64]),
+    (9, 1, 1031, 1025, [8, 16, 1]),
+    (7, 3, 2050, 2049, [100, 5, 64]),
+    (3, 20, 64, 48, [256, 255, 31]),
+    (3, 5, 40, 24, [300, 7]),
+    (600, 1, 65, 3000, [16, 8]),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,row_len,K,N,ranks", CASES)
+@pytest.mark.parametrize("aligned", [True, False])
+def test_row_kernel_edges_match_the_oracle(gpu, dtype, rows, row_len, K, N, ranks, aligned):
+    print("case:", dtype, rows, row_len, K, N, ranks, aligned, flush=True)
+    g = torch.Generator().manual_seed(rows * 1000 + K + N)
+    # weights N(0, 0.02): |t| stays near 0.02 * sqrt(K) < 1 and the delta near 2 * 0.02 * |t| * sqrt(rank) < 1, so that
+    # fp32 sums in two orders differ by at most some sqrt(terms) * 2^-24 < 4e-6, inside the fp32 tolerance of 1e-5
+    # (with N(0, 0.1) both factors grow five times and two fp32 orders differ by up to 25 times as much)
+    adapters = {f"a{i}": {"m": peft_layer(g, K, N, r, 2.0 * r)} for i, r in enumerate(ranks)}
+    cache = make_cache(adapters, {"m": (K, N)}, len(ranks), max(ranks), gpu, dtype, tiled=False)
+    ids = list(adapters) + ["__base__"]
+    row_slot = cache.ensure_resident([ids[i] for i in torch.randint(0, len(ids), (rows,), generator=g).tolist()])
+    seq = torch.randint(0, row_len + 2, (rows,), generator=g, dtype=torch.int32)
+    seq[0] = row_len
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    base = torch.randn(rows, row_len, N, generator=g).to(dtype)
+    pad = 0 if aligned else 1
+
+    def strided(t):
+        flat = t.view(-1, t.shape[-1])
+        big = torch.full((flat.shape[0] + 1, flat.shape[1] + 2 * pad), 7.0, dtype=dtype, device=gpu)
+        out = big.view(-1)[pad:].as_strided(flat.shape, (big.shape[1], 1))
+        out.copy_(flat)
+        return out, big
+
+    dx, _ = strided(x)
+    dy, around = strided(base)
+    sgmv.lora_apply_rows(dx, dy, cache, "m", row_slot, seq.to(gpu), row_len)
+    A, B, rk, sc = oracle_slot_tensors(cache, adapters, "m", dtype)
+    want = reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc)
+    torch.testing.assert_close(dy.cpu().view(rows, row_len, N), want, **tol_for(dtype))
+    untouched = torch.tensor([[int(s) == 0 or m >= int(n) for m in range(row_len)] for s, n in zip(row_slot.tolist(), seq)])
+    assert torch.equal(dy.cpu().view(rows, row_len, N)[untouched], base[untouched])
+    if not aligned:  # nothing between or around the rows was written
+        gaps = torch.ones(around.numel(), dtype=torch.bool)
+        gaps[1:].as_strided(dy.shape, dy.stride()).fill_(False)
+        assert torch.equal(around.view(-1).cpu()[gaps], torch.full((int(gaps.sum()),), 7.0, dtype=dtype))
