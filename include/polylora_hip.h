@@ -38,6 +38,9 @@
  *                          launch (both Triton kernels of layers.py:45-53)
  *   pl_lora_fused_stacked <- the same for sibling Linears in one launch
  *                          (sgmv.py:141-175 stack_num reads x once)
+ *   pl_lora_long_stacked <- the same in two launches, for more data or
+ *                          higher ranks than one launch suits
+ *   pl_lora_long_workspace_bytes (size of its workspaces)
  *   pl_slot_upload      <- src/polylora/cache.py:119-150 _load_adapter_into_slot
  *                          (host->device copy of one adapter into a slot)
  *   pl_host_copy_async  <- the same for an image in pageable memory: its
@@ -108,6 +111,9 @@ typedef struct pl_group {
 
 /* Modules one pl_sgmv_shrink_stacked launch can serve. */
 #define PL_MAX_STACKED_MODULES 4
+
+/* Largest slot rank capacity pl_lora_long_stacked takes (half of it in fp32). */
+#define PL_LONG_MAX_RANK 256
 
 /* Maximum slot count accepted by pl_plan_build (slot 0 included). */
 #define PL_MAX_SLOTS 4096
@@ -317,6 +323,23 @@ int pl_lora_fused_stacked(int32_t dtype, const void* x, int64_t ldx, int32_t K, 
                           int32_t num_modules, int32_t ldt, const int32_t* tok,
                           const pl_group* groups, const int32_t* meta, int64_t group_cap,
                           int32_t group_tokens, int32_t slices, int32_t epilogue, void* stream);
+
+/* The same operation as pl_lora_fused_stacked in two launches, a shrink into
+ * a workspace of the caller and an expand, for long segments and ranks up to
+ * PL_LONG_MAX_RANK (half of it in fp32).  `tokens` is the plan's token
+ * capacity (rows * row_len); ws[j] is module j's own workspace, 16-byte
+ * aligned, of ws_bytes >= pl_lora_long_workspace_bytes(dtype, tokens, ldt)
+ * bytes, its contents ignored and overwritten: two calls that may overlap on
+ * the GPU need workspaces of their own. */
+int64_t pl_lora_long_workspace_bytes(int32_t dtype, int64_t tokens, int32_t ldt);
+int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, int32_t K, int32_t n_modules,
+                         const int32_t* modules, void* const* y, const int64_t* ldy,
+                         const int32_t* N, const void* arena, const pl_slot_entry* table,
+                         int32_t num_modules, int32_t ldt, const int32_t* tok,
+                         const pl_group* groups, const int32_t* meta, int64_t group_cap,
+                         int32_t group_tokens, int64_t tokens, void* const* ws, int64_t ws_bytes,
+                         int32_t epilogue, void* stream);
+
 
 /* Row-based LoRA on the slot arena for shapes the tiled path rejects
  * (any K, N, strides, alignment).  Writes y[b*row_len+m] for m < seq_len[b].

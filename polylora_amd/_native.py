@@ -75,6 +75,11 @@ _SIGNATURES: dict[str, tuple] = {
         c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_void_p, c_int64, c_int32, c_int64,
         c_int32, c_int32, c_void_p,
     ),
+    "pl_lora_long_workspace_bytes": (c_int32, c_int64, c_int32),
+    "pl_lora_long_stacked": (
+        c_int32, c_void_p, c_int64, c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+        c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int64, c_void_p, c_int64, c_int32, c_void_p,
+    ),
     "pl_lora_fused": (
         c_int32, c_void_p, c_int64, c_int32, c_void_p, c_int64, c_int32, c_void_p, c_void_p, c_int32,
         c_int32, c_int32, c_void_p, c_void_p, c_void_p, c_int64, c_int32, c_int32, c_int32, c_void_p,

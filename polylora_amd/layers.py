@@ -102,7 +102,9 @@ class MultiLoraLinear(nn.Module):
             return None
         plan = self._plan(lora_ctx, rows, row_len, seq_lens, weight_indices)
         main = sgmv._stream(x.device)  # handle of the caller's stream
-        fused = sgmv.fused_ok(plan, cache, in_features)
+        # ranks above the fused kernel's: the two-launch path alone
+        long = cache.rank8_cap > sgmv.FUSED_MAX_RANK and sgmv.long_ok(plan, cache, in_features, self._n_out)
+        fused = long or sgmv.fused_ok(plan, cache, in_features)
         run_out = self._run_forward(x, x2, plan, lora_ctx, reshape, main, fused)
         if run_out is not None:
             return run_out
@@ -115,12 +117,15 @@ class MultiLoraLinear(nn.Module):
             sgmv.lora_decode_stacked(x2, [y2], cache, [self.module_name], plan, stream=main)
             return base_3d.reshape(base.shape)
         if fused:
-            # long adapter segments: base GEMM, then one fused shrink+expand launch
+            # long adapter segments: base GEMM, then one fused shrink+expand
+            # launch, or two where its size or the ranks ask for them
             self._observe_call(x, _version_of(x), lora_ctx.stack)
             base = self.base_layer(x)
             base_3d = reshape(base)
             y2 = base_3d.view(rows * row_len, base_3d.shape[-1])
-            if y2.shape[1] == self._n_out and y2.dtype == cache.dtype and y2.data_ptr() % 16 == 0:
+            if long:
+                sgmv.lora_long_stacked(x2, [y2], cache, [self.module_name], plan)
+            elif y2.shape[1] == self._n_out and y2.dtype == cache.dtype and y2.data_ptr() % 16 == 0:
                 # x2 passed tiled_shapes_ok and y2 is the fresh contiguous base output
                 sgmv._fused_launch(x2, y2, cache, self.module_name, plan, _native.PL_EPI_FALLBACK, None, main)
             else:
@@ -186,11 +191,14 @@ class MultiLoraLinear(nn.Module):
         done = fused  # the outputs are complete after the launches below
         if fused:
             # long adapter segments: every sibling's base GEMM, then one fused
-            # launch for all of them
+            # launch (or the two-launch path) for all of them
             bases = [m.base_layer(x) for m in siblings]
             outs = [reshape(b) for b in bases]
-            sgmv.lora_fused_stacked(x2, [o.view(tokens, o.shape[-1]) for o in outs], cache, list(run), plan,
-                                    stream=main)
+            ys = [o.view(tokens, o.shape[-1]) for o in outs]
+            if cache.rank8_cap > sgmv.FUSED_MAX_RANK:
+                sgmv.lora_long_stacked(x2, ys, cache, list(run), plan)
+            else:
+                sgmv.lora_fused_stacked(x2, ys, cache, list(run), plan, stream=main)
         elif tokens >= OVERLAP_MIN_TOKENS:
             main_s = torch.cuda.current_stream(x.device)
             side = sgmv.side_stream(x.device)

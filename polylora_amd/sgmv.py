@@ -241,7 +241,9 @@ def lora_apply(
 
     x: [rows*row_len, in_features], y: [rows*row_len, out_features], both of
     the cache's dtype, on the cache's device.  Long adapter segments go to
-    the fused kernel (lora_fused) unless k_splits asks for the split pair;
+    the fused kernel (lora_fused) or, with more data or ranks above its
+    limit, to the two-launch path (long_ok), unless k_splits asks for the
+    split pair;
     x / y that do not meet the tiled path's alignment go to the row-based HIP
     kernels.
     """
@@ -249,10 +251,14 @@ def lora_apply(
     _check_operands(x, y, cache, module_name, plan.tokens_cap)
     if not _tiled_ok(x, y):
         return lora_apply_rows(x, y, cache, module_name, plan.row_slot, plan.seq_lens, plan.row_len, epilogue=epilogue)
-    if k_splits is None and fused_ok(plan, cache, int(x.shape[1])):
-        # operands checked above; fused_ok guarantees the rank limit
-        _fused_launch(x, y, cache, module_name, plan, epilogue, None, _stream(x.device))
-        return y
+    if k_splits is None:
+        # operands checked above; fused_ok and long_ok guarantee the rank limits
+        if fused_ok(plan, cache, int(x.shape[1])):
+            _fused_launch(x, y, cache, module_name, plan, epilogue, None, _stream(x.device))
+            return y
+        if long_ok(plan, cache, x.shape[1], y.shape[1]):
+            _long_launch(x, [y], cache, [module_name], plan, epilogue, _stream(x.device))
+            return y
     lib = _native.load()
     dt = _native.dtype_code(x.dtype)
     K = int(x.shape[1])
@@ -529,6 +535,64 @@ def fused_ok(plan: SgmvPlan, cache, in_features: int) -> bool:
     return plan.tokens_cap >= 64 * max(1, distinct) and plan.tokens_cap >= 1024
 
 
+# Ranks pl_lora_long_stacked takes (half of it in fp32), and the bytes of y
+# it must read and write to win over the fused launch: its second launch
+# costs about 5 us, which its faster streaming pays back from there on.
+# Measured on MI355X (bf16 unless said; y traffic of the plan's capacity,
+# fused against long): 2048 -> 8192 rank 16, 67 MB 16.4 / 19.3 us, 134 MB
+# 32.5 / 28.2; 4096 -> 4096 rank 32, 67 MB 21.0 / 23.3, 134 MB 40.9 / 35.5;
+# 4096 -> 2 x 14336 rank 16, 117 MB 28.4 / 26.3; fp32 768 -> 3072 rank 8,
+# 100 MB 20.6 / 22.5, 201 MB 37.4 / 35.4.  Above rank 64 the other choice is
+# the split pair, slower from 2048 tokens on (4096 -> 4096 rank 128, 1024
+# tokens 19.3 / 21.5 us, 2048 tokens 33.3 / 28.8).
+LONG_MAX_RANK = 256
+LONG_MIN_Y_BYTES = 112 << 20
+LONG_MIN_TOKENS = 2048
+
+
+def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -> bool:
+    """Whether the two-launch path (pl_lora_long_stacked) suits a plan and modules of `out_features` columns in all."""
+    distinct, rank, tokens = plan.distinct_slots, cache.rank8_cap, plan.tokens_cap
+    if distinct is None or tokens < max(1024, 64 * max(1, distinct)):
+        return False
+    es = cache.dtype.itemsize
+    if rank > FUSED_MAX_RANK:
+        return rank <= LONG_MAX_RANK * 2 // max(2, es) and tokens >= LONG_MIN_TOKENS
+    return in_features <= FUSED_MAX_K and 2 * es * tokens * out_features >= LONG_MIN_Y_BYTES
+
+
+def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, out_features: int, stream: int | None) -> bool:
+    """long_ok, on the current stream only: the workspace is allocated there."""
+    return long_ok(plan, cache, x.shape[1], out_features) and stream in (None, _stream(x.device))
+
+
+def _long_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, epilogue: int, stream: int) -> None:
+    """pl_lora_long_stacked on operands the caller has checked, on the current stream `stream`.
+
+    The workspaces come from torch's allocator for this call alone, so calls
+    on other streams or threads never share them.
+    """
+    lib = _native.load()
+    _, mods, (yp, ldy, nn_) = _fused_set(cache, module_names)
+    dt = _native.dtype_code(x.dtype)
+    n = len(ys)
+    arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
+    nbytes = -(-int(lib.pl_lora_long_workspace_bytes(dt, plan.tokens_cap, ldt)) // 256) * 256
+    buf = torch.empty(n * nbytes, dtype=torch.uint8, device=x.device)
+    base = buf.data_ptr()
+    ws = (ctypes.c_void_p * n)(*(base + i * nbytes for i in range(n)))
+    for i, y in enumerate(ys):
+        yp[i] = y.data_ptr()
+        ldy[i] = y.stride(0)
+    _native.check(
+        lib.pl_lora_long_stacked(
+            dt, x.data_ptr(), x.stride(0), x.shape[1], n, mods, yp, ldy, nn_, arena, table, n_mod, ldt,
+            *plan.launch_args, plan.tokens_cap, ws, nbytes, epilogue, stream,
+        ),
+        "pl_lora_long_stacked",
+    )
+
+
 def lora_fused(
     x: torch.Tensor,
     y: torch.Tensor,
@@ -540,7 +604,8 @@ def lora_fused(
     slices: int | None = None,
     stream: int | None = None,
 ) -> torch.Tensor:
-    """y[t] += scale * (x[t] @ A^T) @ B^T for every planned token t, in place, in one launch (pl_lora_fused).
+    """y[t] += scale * (x[t] @ A^T) @ B^T for every planned token t, in place, in one launch (pl_lora_fused),
+    or in two where long_ok prefers them and no slices are asked for.
 
     Same operands as lora_apply; needs the tiled path's alignment and slot
     ranks up to FUSED_MAX_RANK.
@@ -594,6 +659,9 @@ def _fused_launch(x, y, cache, module_name: str, plan: SgmvPlan, epilogue: int, 
     entry point is called without per-argument conversion.
     """
     N = y.shape[1]
+    if slices is None and _use_long(x, plan, cache, N, stream):
+        _long_launch(x, [y], cache, [module_name], plan, epilogue, stream)
+        return
     c32 = _native.c32
     rc = _native.raw("pl_lora_fused")(
         c32(_native.dtype_code(x.dtype)), ctypes.c_void_p(x.data_ptr()), ctypes.c_int64(x.stride(0)),
@@ -618,7 +686,33 @@ def lora_fused_stacked(
     """lora_fused for sibling Linears fed the same x, in one launch (pl_lora_fused_stacked): ys[i] in place.
 
     A tile's modules run side by side on one XCD, so x comes from HBM once.
+    As lora_fused, in two launches where long_ok prefers them.
     """
+    _check_stacked(x, ys, cache, module_names, plan)
+    if cache.rank8_cap > FUSED_MAX_RANK:
+        raise ValueError(f"lora_fused takes ranks up to {FUSED_MAX_RANK}; the cache holds up to {cache.rank8_cap}")
+    if slices is None and _use_long(x, plan, cache, sum(y.shape[1] for y in ys), stream):
+        _long_launch(x, ys, cache, module_names, plan, epilogue, _stream(x.device))
+        return ys
+    specs, mods, (yp, ldy, nn_) = _fused_set(cache, module_names)
+    for i, y in enumerate(ys):
+        yp[i] = y.data_ptr()
+        ldy[i] = y.stride(0)
+    n_slices = slices if slices is not None else choose_slices(plan, min(spec.out_features for spec in specs))
+    arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
+    _native.check(
+        _native.load().pl_lora_fused_stacked(
+            _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], len(ys), mods, yp, ldy, nn_,
+            arena, table, n_mod, ldt, *plan.launch_args, n_slices, epilogue,
+            _stream(x.device) if stream is None else stream,
+        ),
+        "pl_lora_fused_stacked",
+    )
+    return ys
+
+
+def _check_stacked(x: torch.Tensor, ys: list, cache, module_names: list, plan: SgmvPlan) -> None:
+    """Operand checks of the stacked launches over long segments."""
     _require_gpu(x, "lora_fused_stacked")
     n = len(module_names)
     if not 1 <= n <= _native.PL_MAX_STACKED_MODULES or len(ys) != n:
@@ -627,7 +721,7 @@ def lora_fused_stacked(
     _check_operands(x, ys[0], cache, module_names[0], plan.tokens_cap)
     if not _tiled_ok(x, ys[0]):
         raise ValueError("lora_fused needs 16-byte aligned rows and K, N multiples of 16 bytes")
-    specs, mods, arrays = _fused_set(cache, module_names)
+    specs, _ = _module_set(cache, module_names)
     chunk = 16 // x.element_size()
     for y, spec in zip(ys[1:], specs[1:]):
         if spec.in_features != x.shape[1]:
@@ -639,22 +733,13 @@ def lora_fused_stacked(
             raise TypeError(f"y {y.dtype} on {y.device} must match the adapter cache ({cache.dtype} on {cache.device})")
         if st[1] != 1 or (shape[1] | st[0]) % chunk or y.data_ptr() % 16:
             raise ValueError("lora_fused needs 16-byte aligned rows and K, N multiples of 16 bytes")
-    if cache.rank8_cap > FUSED_MAX_RANK:
-        raise ValueError(f"lora_fused takes ranks up to {FUSED_MAX_RANK}; the cache holds up to {cache.rank8_cap}")
-    yp, ldy, nn_ = arrays
-    for i, y in enumerate(ys):
-        yp[i] = y.data_ptr()
-        ldy[i] = y.stride(0)
-    n_slices = slices if slices is not None else choose_slices(plan, min(spec.out_features for spec in specs))
-    arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
-    _native.check(
-        _native.load().pl_lora_fused_stacked(
-            _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], n, mods, yp, ldy, nn_,
-            arena, table, n_mod, ldt, *plan.launch_args, n_slices, epilogue,
-            _stream(x.device) if stream is None else stream,
-        ),
-        "pl_lora_fused_stacked",
-    )
+
+
+def lora_long_stacked(x: torch.Tensor, ys: list, cache, module_names: list, plan: SgmvPlan, *,
+                      epilogue: int = _native.PL_EPI_FALLBACK) -> list:
+    """lora_fused_stacked in two launches (pl_lora_long_stacked), for slot ranks up to LONG_MAX_RANK (half in fp32)."""
+    _check_stacked(x, ys, cache, module_names, plan)
+    _long_launch(x, ys, cache, module_names, plan, epilogue, _stream(x.device))
     return ys
 
 

@@ -1,0 +1,102 @@
+"""The two-launch path of long segments (lora_long_stacked) at the edges of its tiles, against the oracle.
+
+Segments around one, two and four 16-token tiles, so that a unit of tiles
+holds one slot or several; K around one wave's step and a turn of the four
+waves; N around an MFMA tile and a workgroup's chunk; ranks around a pass (and
+two passes, above 64); a second module that some adapters do not have; plans
+of 16- and 64-token groups, and one with enough tiles for the two-tile shrink.
+
+Reference: the fallback of layers.py:112-134 (reference_forward).
+"""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+from oracle.lora import reference_forward
+from polylora_amd import sgmv
+from tests._util import make_cache, oracle_slot_tensors, peft_layer, tol_for
+
+pytestmark = pytest.mark.gpu
+
+CASES = [
+    # rows, row_len, K, (N of the two modules), ranks
+    (3, 1, 8, (8, 16), [1, 2]),
+    (9, 15, 64, (520, 8), [8, 16, 3]),
+    (6, 17, 264, (504, 512), [16, 15]),
+    (5, 65, 256, (1032, 24), [17, 32, 33]),
+    (12, 33, 1000, (136, 264), [64, 5]),
+    (4, 100, 520, (72, 640), [65, 128, 16]),
+    (17, 16, 72, (48, 56), [40, 9, 1, 24]),
+    (40, 256, 136, (264, 16), [16, 31, 64]),
+    (3, 50, 128, (88, 16), [256, 129, 70]),
+]
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("group_tokens", [16, 64])
+@pytest.mark.parametrize("rows,row_len,K,Ns,ranks", CASES)
+def test_long_path_edges_match_the_oracle(gpu, dtype, group_tokens, rows, row_len, K, Ns, ranks):
+    print("case:", dtype, group_tokens, rows, row_len, K, Ns, ranks, flush=True)
+    if dtype == torch.float32 and max(ranks) > sgmv.LONG_MAX_RANK // 2:
+        ranks = [min(r, sgmv.LONG_MAX_RANK // 2) for r in ranks]
+    g = torch.Generator().manual_seed(rows * 1000 + K + Ns[0])
+    # weights N(0, 0.02): |t| and the deltas stay near 1 or below, so that fp32 sums in two orders differ by at most
+    # some sqrt(terms) * 2^-24 < 4e-6, inside the fp32 tolerance of 1e-5
+    adapters = {}
+    for i, r in enumerate(ranks):
+        adapters[f"a{i}"] = {"m0": peft_layer(g, K, Ns[0], r, 2.0 * r)}
+        if i % 2 == 0:
+            adapters[f"a{i}"]["m1"] = peft_layer(g, K, Ns[1], max(1, r // 2), 1.0 * r)
+    cache = make_cache(adapters, {"m0": (K, Ns[0]), "m1": (K, Ns[1])}, len(ranks), max(ranks), gpu, dtype)
+    ids = list(adapters) + ["__base__"]
+    row_slot = cache.ensure_resident([ids[i] for i in torch.randint(0, len(ids), (rows,), generator=g).tolist()])
+    seq = torch.randint(0, row_len + 2, (rows,), generator=g, dtype=torch.int32)
+    seq[0] = row_len
+    plan = sgmv.SgmvPlan(row_slot, seq.to(gpu), row_len, cache.num_slots, distinct_slots=len(ranks),
+                         group_tokens=group_tokens)
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    bases = [torch.randn(rows, row_len, n, generator=g).to(dtype) for n in Ns]
+    dx = x.to(gpu).view(-1, K)
+    for epilogue in (0, 1):
+        # the modules one by one, then stacked, with bit-equal outputs
+        one = [b.to(gpu).view(-1, b.shape[-1]) for b in bases]
+        both = [t.clone() for t in one]
+        for name, y in zip(("m0", "m1"), one):
+            sgmv.lora_long_stacked(dx, [y], cache, [name], plan, epilogue=epilogue)
+        sgmv.lora_long_stacked(dx, both, cache, ["m0", "m1"], plan, epilogue=epilogue)
+        assert all(torch.equal(a, b) for a, b in zip(one, both))
+        for name, y, base in zip(("m0", "m1"), both, bases):
+            got = y.cpu().view(base.shape)
+            A, B, rk, sc = oracle_slot_tensors(cache, adapters, name, dtype)
+            torch.testing.assert_close(got, reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc), **tol_for(dtype))
+            keep = torch.tensor([[int(rk[s]) == 0 or m >= int(n) for m in range(row_len)]
+                                 for s, n in zip(row_slot.tolist(), seq)])
+            assert torch.equal(got[keep], base[keep])
+
+
+def test_the_dispatch_takes_the_long_path_where_its_rule_says(gpu, monkeypatch):
+    """lora_apply and lora_fused_stacked go through it for large outputs and for high ranks, and only there."""
+    calls = []
+    launch = sgmv._long_launch
+    monkeypatch.setattr(sgmv, "_long_launch", lambda x, ys, *a: (calls.append(len(ys)), launch(x, ys, *a))[1])
+    g = torch.Generator().manual_seed(5)
+    for rank, rows, n, want in ((16, 20, 1024, []), (16, 20, 17000, [1, 1]), (96, 20, 64, [1]), (96, 8, 64, [])):
+        adapters = {"a": {"m": peft_layer(g, 64, n, rank, 2.0 * rank)}}
+        cache = make_cache(adapters, {"m": (64, n)}, 1, rank, gpu, torch.bfloat16)
+        row_slot = cache.ensure_resident(["a"] * rows)
+        seq = torch.full((rows,), 128, dtype=torch.int32)
+        plan = sgmv.SgmvPlan(row_slot, seq.to(gpu), 128, cache.num_slots, distinct_slots=1)
+        x, base = (torch.randn(rows, 128, k, generator=g).bfloat16() for k in (64, n))
+        A, B, rk, sc = oracle_slot_tensors(cache, adapters, "m", torch.bfloat16)
+        ref = reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc)
+        calls.clear()
+        ops = [lambda x, y: sgmv.lora_apply(x, y, cache, "m", plan)]
+        if rank <= sgmv.FUSED_MAX_RANK:  # lora_fused_stacked refuses higher ranks
+            ops.append(lambda x, y: sgmv.lora_fused_stacked(x, [y], cache, ["m"], plan))
+        for op in ops:
+            y = base.to(gpu).view(-1, n)
+            op(x.to(gpu).view(-1, 64), y)
+            torch.testing.assert_close(y.cpu().view(base.shape), ref, **tol_for(torch.bfloat16))
+        assert calls == want, (rank, rows, n)
