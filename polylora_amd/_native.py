@@ -125,7 +125,7 @@ _SIGNATURES: dict[str, tuple] = {
 }
 _RESTYPES = {"pl_last_error": ctypes.c_char_p, "pl_plan_group_capacity": c_int64, "pl_shrink_workspace_bytes": c_int64,
              "pl_host_alloc": c_void_p, "pl_sgmv_ref_workspace_bytes": c_int64, "pl_decode_counter_ints": c_int64,
-             "pl_sgmv_ref_part_bytes": c_int64}
+             "pl_sgmv_ref_part_bytes": c_int64, "pl_lora_long_workspace_bytes": c_int64}
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 

@@ -601,3 +601,12 @@ def test_operator_part_sizes_depend_only_on_what_their_keys_hold():
     assert size(bf, 1, 256, 1, 64, 1001, 65, 0) == 0  # N not whole 16-byte chunks
     # the expand reads the caller's intermediate directly: no scratch; the shrink's split planes need some
     assert size(bf, 1, 256, 1, 64, 1000, 65, 2) == 0 and size(bf, 0, 256, 1, 4096, 64, 65, 2) > 0
+
+
+def test_long_workspace_size_is_64_bit():
+    """The long path's workspace size past 2 GiB, and its rank limits."""
+    lib = _native.load()
+    assert lib.pl_lora_long_workspace_bytes(_native.PL_BF16, 1 << 26, 256) == (1 << 26) * 256 * 2
+    assert lib.pl_lora_long_workspace_bytes(_native.PL_F32, 3, 40) == 3 * 64 * 4  # rows of whole 32-rank blocks
+    assert lib.pl_lora_long_workspace_bytes(_native.PL_BF16, 8, 264) == 0
+    assert lib.pl_lora_long_workspace_bytes(_native.PL_F32, 8, 136) == 0
