@@ -8,12 +8,14 @@ torch is imported first so that the library binds to torch's HIP runtime.
 from __future__ import annotations
 
 import ctypes
+import importlib.machinery
 from ctypes import c_int32, c_int64, c_void_p
 from pathlib import Path
 
 import torch  # noqa: F401  (loads the HIP runtime the library must share)
 
 LIB_PATH = Path(__file__).resolve().parent / "_lib" / "libpolylora_hip.so"
+CALLS_PATH = LIB_PATH.parent / "_calls.so"
 
 PL_F32, PL_BF16, PL_F16 = 0, 1, 2
 PL_OK, PL_ERR_ARG, PL_ERR_ALIGN, PL_ERR_LAUNCH, PL_ERR_LIMIT = 0, 1, 2, 3, 4
@@ -130,37 +132,8 @@ _RESTYPES = {"pl_last_error": ctypes.c_char_p, "pl_plan_group_capacity": c_int64
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 
 _lib = None
+_calls = None
 _checked_runtime = False
-
-
-_raw: dict = {}
-
-
-def raw(name: str):
-    """Entry point `name` without ctypes argument conversion.
-
-    Every argument must already be a ctypes object of the declared type
-    (c_int32, c_int64, c_void_p); arguments that do not change between calls
-    can then be built once and passed as they are, which saves the per-call
-    conversion of the declared-argtypes binding.  Returns int32.
-    """
-    f = _raw.get(name)
-    if f is None:
-        f = load()[name]  # a separate function object with no argtypes
-        f.restype = c_int32
-        _raw[name] = f
-    return f
-
-
-_c32: dict = {}
-
-
-def c32(v: int) -> ctypes.c_int32:
-    """A shared c_int32 for a small constant argument (dtype codes, flags, counts)."""
-    got = _c32.get(v)
-    if got is None:
-        got = _c32[v] = c_int32(v)
-    return got
 
 
 class NativeLibraryMissing(RuntimeError):
@@ -184,6 +157,21 @@ def load() -> ctypes.CDLL:
         fn.restype = _RESTYPES.get(name, c_int32)
     _lib = lib
     return lib
+
+
+def calls():
+    """The library's per-call functions as CPython entry points (csrc/pycalls.cpp): the C functions' arguments in
+    their order as ints (None for a null pointer, a tuple for a host array of per-module values); each returns the
+    status for ``check``."""
+    global _calls
+    if _calls is None:
+        load()  # the one instance of the library both bindings use
+        if not CALLS_PATH.exists():
+            raise NativeLibraryMissing(f"{CALLS_PATH} not found; build it with `python -m polylora_amd.build`")
+        loader = importlib.machinery.ExtensionFileLoader("_calls", str(CALLS_PATH))
+        _calls = loader.create_module(importlib.machinery.ModuleSpec("_calls", loader, origin=str(CALLS_PATH)))
+        loader.exec_module(_calls)
+    return _calls
 
 
 def check(status: int, what: str) -> None:

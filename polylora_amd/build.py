@@ -1,6 +1,8 @@
 """Build the gfx950 HIP library ``polylora_amd/_lib/libpolylora_hip.so``.
 
-Run ``python -m polylora_amd.build``.  Every source under ``csrc/`` is
+Run ``python -m polylora_amd.build``.  Also builds ``_lib/_calls.so``, the
+CPython entry points of the per-call functions (``csrc/pycalls.cpp``), linked
+against the library.  Every source under ``csrc/`` is
 compiled with ``hipcc --offload-arch=gfx950`` into an object under
 ``polylora_amd/_build/`` and the objects are linked into one shared library
 with a plain C ABI (``include/polylora_hip.h``); nothing links against
@@ -14,6 +16,7 @@ import os
 import shutil
 import subprocess
 import sys
+import sysconfig
 from pathlib import Path
 
 PACKAGE_DIR = Path(__file__).resolve().parent
@@ -21,6 +24,7 @@ CSRC_DIR = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIB_DIR = PACKAGE_DIR / "_lib"
 LIB_PATH = LIB_DIR / "libpolylora_hip.so"
+CALLS_PATH = LIB_DIR / "_calls.so"
 INCLUDE_DIR = PACKAGE_DIR.parent / "include"
 
 ARCH = "gfx950"
@@ -90,9 +94,22 @@ def build(verbose: bool = False) -> Path:
     if proc.returncode != 0:
         raise RuntimeError(f"link failed: {' '.join(link)}\n{proc.stdout}")
     os.replace(tmp_lib, LIB_PATH)
+    _build_calls(hipcc)
     if verbose:
         print(f"built {LIB_PATH}")
     return LIB_PATH
+
+
+def _build_calls(hipcc: str) -> None:
+    """csrc/pycalls.cpp, host code only, for the running interpreter."""
+    cxx = [found] if (found := shutil.which("g++")) else [hipcc, "-x", "c++"]
+    tmp = CALLS_PATH.with_suffix(".so.tmp")
+    cmd = [*cxx, "-O2", "-fPIC", "-std=c++17", "-Wall", "-shared", f"-I{sysconfig.get_paths()['include']}",
+           str(CSRC_DIR / "pycalls.cpp"), "-o", str(tmp), f"-L{LIB_DIR}", "-lpolylora_hip", "-Wl,-rpath,$ORIGIN"]
+    proc = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"build failed: {' '.join(cmd)}\n{proc.stdout}")
+    os.replace(tmp, CALLS_PATH)
 
 
 if __name__ == "__main__":

@@ -19,7 +19,6 @@ There is no CPU path: CPU tensors raise.
 from __future__ import annotations
 
 import ctypes
-import threading
 
 import torch
 
@@ -82,7 +81,7 @@ class SgmvPlan:
     """
 
     __slots__ = ("rows", "row_len", "num_slots", "group_tokens", "tokens_cap", "group_cap", "tok", "groups", "meta",
-                 "row_slot", "seq_lens", "distinct_slots", "launch_args", "launch_args_c", "active", "_build")
+                 "row_slot", "seq_lens", "distinct_slots", "launch_args", "active", "_build")
 
     def __init__(self, row_slot: torch.Tensor, seq_lens: torch.Tensor, row_len: int, num_slots: int,
                  distinct_slots: int | None = None, group_tokens: int | None = None,
@@ -116,9 +115,6 @@ class SgmvPlan:
         # the plan's arguments of the fused entry points, in their order
         self.launch_args = (self.tok.data_ptr(), self.groups.data_ptr(), self.meta.data_ptr(), max(1, self.group_cap),
                             self.group_tokens)
-        self.launch_args_c = (ctypes.c_void_p(self.launch_args[0]), ctypes.c_void_p(self.launch_args[1]),
-                              ctypes.c_void_p(self.launch_args[2]), ctypes.c_int64(self.launch_args[3]),
-                              ctypes.c_int32(self.launch_args[4]))
         self.row_slot, self.seq_lens, self.active = row_slot, seq_lens, active
         out = (self.tok.data_ptr(), self.groups.data_ptr(), self.meta.data_ptr(), max(1, self.group_cap))
         if active is None:
@@ -259,44 +255,20 @@ def lora_apply(
         if long_ok(plan, cache, x.shape[1], y.shape[1]):
             _long_launch(x, [y], cache, [module_name], plan, epilogue, _stream(x.device))
             return y
-    lib = _native.load()
     dt = _native.dtype_code(x.dtype)
-    K = int(x.shape[1])
-    N = int(y.shape[1])
-    ldt = cache.rank8_cap
+    K = x.shape[1]
+    arena, table, n_mod, column, ldt = _cache_args(cache, module_name)
     stream = _stream(x.device)
     rows = max(1, plan.tokens_cap)
-    group_cap = max(1, plan.group_cap)
-    splits, _, nbytes = _shrink_geometry(lib, dt, K, x.dtype, plan, rows, ldt, k_splits)
+    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, x.dtype, plan, rows, ldt, k_splits)
     ws = _workspace(x.device, stream)
     buf = ws.get(nbytes)
     ws.owner = None  # planes of an earlier separate shrink on this workspace are gone
-    status = lib.pl_lora_apply(
-        dt,
-        x.data_ptr(),
-        x.stride(0),
-        K,
-        y.data_ptr(),
-        y.stride(0),
-        N,
-        cache.arena.data_ptr(),
-        cache.table.data_ptr(),
-        len(cache.module_index),
-        cache.module_index[module_name],
-        plan.tok.data_ptr(),
-        plan.groups.data_ptr(),
-        plan.meta.data_ptr(),
-        group_cap,
-        plan.group_tokens,
-        buf.data_ptr(),
-        buf.numel(),
-        ldt,
-        rows,
-        splits,
-        epilogue,
-        stream,
-    )
-    _native.check(status, "pl_lora_apply")
+    rc = _native.calls().pl_lora_apply(
+        dt, x.data_ptr(), x.stride(0), K, y.data_ptr(), y.stride(0), y.shape[1], arena, table, n_mod, column,
+        *plan.launch_args, buf.data_ptr(), buf.numel(), ldt, rows, splits, epilogue, stream)
+    if rc:
+        _native.check(rc, "pl_lora_apply")
     return y
 
 
@@ -305,7 +277,7 @@ class ShrinkResult:
 
     ``valid`` turns False once a later shrink has reused that workspace.
     ``batch`` identifies the stacked shrink this result came from (its
-    workspace pointer array) and ``index`` its position in it.
+    workspace addresses) and ``index`` its position in it.
     """
 
     __slots__ = ("ws", "buf", "planes", "rows", "ldt", "plan", "K", "batch", "index")
@@ -321,7 +293,7 @@ class ShrinkResult:
 
 
 class _ShrinkBatch:
-    """The modules of one stacked shrink: their count and workspace pointers as passed to the kernel."""
+    """The modules of one stacked shrink: their count and workspace addresses as passed to the kernel."""
 
     __slots__ = ("n", "ptrs")
 
@@ -380,39 +352,21 @@ def lora_shrink(x: torch.Tensor, cache, module_name: str, plan: SgmvPlan, *, k_s
 
 
 def _module_set(cache, module_names) -> tuple:
-    """(specs, ctypes int32 array of table columns) of a module list, built once per cache and list."""
+    """(specs, table columns, output widths, input width or -1 where they differ) of a module list, built once per
+    cache and list."""
     sets = cache.__dict__.setdefault("_module_sets", {})
     key = tuple(module_names)
     hit = sets.get(key)
-    if hit is not None:
-        return hit
-    specs = []
-    for name in module_names:
-        spec = cache.module_specs.get(name)
-        if spec is None:
-            raise KeyError(f"module {name!r} is not in the adapter cache")
-        specs.append(spec)
-    cols = (ctypes.c_int32 * len(specs))(*(cache.module_index[name] for name in module_names))
-    sets[key] = (specs, cols)
-    return specs, cols
-
-
-def _fused_set(cache, module_names) -> tuple:
-    """_module_set plus the output-pointer, row-stride and column-count arrays of one stacked fused launch.
-
-    The arrays are reused call after call by the calling thread (the pointers
-    and strides are rewritten before each launch, which reads them when it is
-    enqueued); another thread gets its own, since the library call runs
-    without the GIL.
-    """
-    sets = cache.__dict__.setdefault("_fused_sets", {})
-    key = (tuple(module_names), threading.get_ident())
-    hit = sets.get(key)
     if hit is None:
-        specs, cols = _module_set(cache, module_names)
-        n = len(specs)
-        cnt = (ctypes.c_int32 * n)(*(spec.out_features for spec in specs))
-        hit = sets[key] = (specs, cols, ((ctypes.c_void_p * n)(), (ctypes.c_int64 * n)(), cnt))
+        specs = []
+        for name in key:
+            spec = cache.module_specs.get(name)
+            if spec is None:
+                raise KeyError(f"module {name!r} is not in the adapter cache")
+            specs.append(spec)
+        widths = {spec.in_features for spec in specs}
+        hit = sets[key] = (specs, tuple(cache.module_index[name] for name in key),
+                           tuple(spec.out_features for spec in specs), widths.pop() if len(widths) == 1 else -1)
     return hit
 
 
@@ -420,19 +374,19 @@ _WS_SETS: dict = {}
 
 
 def _workspace_set(device: torch.device, stream: int, n: int, nbytes: int) -> tuple:
-    """(workspaces, buffers, ctypes pointer array) of positions 0..n-1 of (device, stream)."""
+    """(workspaces, buffers, their addresses, smallest size) of positions 0..n-1 of (device, stream)."""
     key = (device.index if device.index is not None else torch.cuda.current_device(), stream, n)
     hit = _WS_SETS.get(key)
-    if hit is None:
-        wss = [_workspace(device, stream, i) for i in range(n)]
-        hit = [wss, None, None]
-        _WS_SETS[key] = hit
-    wss = hit[0]
+    if hit is not None and hit[3] >= nbytes:
+        for ws, buf in zip(hit[0], hit[1]):
+            if ws.buf is not buf:  # replaced through another set
+                break
+        else:
+            return hit
+    wss = hit[0] if hit is not None else [_workspace(device, stream, i) for i in range(n)]
     bufs = [ws.get(nbytes) for ws in wss]
-    if hit[1] is None or any(b is not c for b, c in zip(bufs, hit[1])):
-        hit[1] = bufs
-        hit[2] = (ctypes.c_void_p * n)(*(b.data_ptr() for b in bufs))
-    return wss, hit[1], hit[2]
+    hit = _WS_SETS[key] = (wss, bufs, tuple(b.data_ptr() for b in bufs), min(b.numel() for b in bufs))
+    return hit
 
 
 def lora_shrink_stacked(x: torch.Tensor, cache, module_names: list, plan: SgmvPlan, *,
@@ -446,9 +400,9 @@ def lora_shrink_stacked(x: torch.Tensor, cache, module_names: list, plan: SgmvPl
     n = len(module_names)
     if not 1 <= n <= _native.PL_MAX_STACKED_MODULES:
         raise ValueError(f"a shrink serves 1..{_native.PL_MAX_STACKED_MODULES} modules, got {n}")
-    specs, modules = _module_set(cache, module_names)
-    K = int(x.shape[1]) if x.dim() == 2 else -1
-    if x.dim() != 2 or x.shape[0] != plan.tokens_cap or any(sp.in_features != K for sp in specs):
+    _, modules, _, fin = _module_set(cache, module_names)
+    K = x.shape[1] if x.dim() == 2 else -1
+    if K < 0 or x.shape[0] != plan.tokens_cap or K != fin:
         raise ValueError(f"x must be [{plan.tokens_cap}, in_features] for every module, got {list(x.shape)}")
     if x.dtype != cache.dtype or x.device != cache.device:
         raise TypeError(f"x {x.dtype} on {x.device} must match the adapter cache ({cache.dtype} on {cache.device})")
@@ -459,15 +413,13 @@ def lora_shrink_stacked(x: torch.Tensor, cache, module_names: list, plan: SgmvPl
         stream = _stream(x.device)
     rows = max(1, plan.tokens_cap)
     splits, planes, nbytes = _shrink_geometry(lib, dt, K, x.dtype, plan, rows, ldt, k_splits)
-    wss, bufs, ptrs = _workspace_set(x.device, stream, n, nbytes)
-    _native.check(
-        lib.pl_sgmv_shrink_stacked(
-            dt, x.data_ptr(), x.stride(0), K, cache.arena.data_ptr(), cache.table.data_ptr(), len(cache.module_index),
-            n, modules, ptrs, plan.tok.data_ptr(), plan.groups.data_ptr(), plan.meta.data_ptr(),
-            max(1, plan.group_cap), plan.group_tokens, min(b.numel() for b in bufs), ldt, rows, splits, stream,
-        ),
-        "pl_sgmv_shrink_stacked",
-    )
+    wss, bufs, ptrs, size = _workspace_set(x.device, stream, n, nbytes)
+    arena, table, n_mod, _, _ = _cache_args(cache, module_names[0])
+    rc = _native.calls().pl_sgmv_shrink_stacked(
+        dt, x.data_ptr(), x.stride(0), K, arena, table, n_mod, n, modules, ptrs, *plan.launch_args, size, ldt, rows,
+        splits, stream)
+    if rc:
+        _native.check(rc, "pl_sgmv_shrink_stacked")
     batch = _ShrinkBatch(n, ptrs)
     return [ShrinkResult(ws, b, planes, rows, ldt, plan, K, batch, i) for i, (ws, b) in enumerate(zip(wss, bufs))]
 
@@ -572,25 +524,19 @@ def _long_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, epilogu
     The workspaces come from torch's allocator for this call alone, so calls
     on other streams or threads never share them.
     """
-    lib = _native.load()
-    _, mods, (yp, ldy, nn_) = _fused_set(cache, module_names)
+    _, mods, widths, _ = _module_set(cache, module_names)
     dt = _native.dtype_code(x.dtype)
     n = len(ys)
     arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
-    nbytes = -(-int(lib.pl_lora_long_workspace_bytes(dt, plan.tokens_cap, ldt)) // 256) * 256
+    nbytes = -(-int(_native.load().pl_lora_long_workspace_bytes(dt, plan.tokens_cap, ldt)) // 256) * 256
     buf = torch.empty(n * nbytes, dtype=torch.uint8, device=x.device)
     base = buf.data_ptr()
-    ws = (ctypes.c_void_p * n)(*(base + i * nbytes for i in range(n)))
-    for i, y in enumerate(ys):
-        yp[i] = y.data_ptr()
-        ldy[i] = y.stride(0)
-    _native.check(
-        lib.pl_lora_long_stacked(
-            dt, x.data_ptr(), x.stride(0), x.shape[1], n, mods, yp, ldy, nn_, arena, table, n_mod, ldt,
-            *plan.launch_args, plan.tokens_cap, ws, nbytes, epilogue, stream,
-        ),
-        "pl_lora_long_stacked",
-    )
+    rc = _native.calls().pl_lora_long_stacked(
+        dt, x.data_ptr(), x.stride(0), x.shape[1], n, mods, tuple([y.data_ptr() for y in ys]),
+        tuple([y.stride(0) for y in ys]), widths, arena, table, n_mod, ldt, *plan.launch_args, plan.tokens_cap,
+        tuple([base + i * nbytes for i in range(n)]), nbytes, epilogue, stream)
+    if rc:
+        _native.check(rc, "pl_lora_long_stacked")
 
 
 def lora_fused(
@@ -652,22 +598,16 @@ def _cache_args_c(cache, module_name: str) -> tuple:
 
 
 def _fused_launch(x, y, cache, module_name: str, plan: SgmvPlan, epilogue: int, slices, stream: int) -> None:
-    """pl_lora_fused on operands the caller has checked.
-
-    The wrapped Linear's hot call: the cache's and the plan's arguments are
-    ctypes objects built once (per cache and module, per plan), and the
-    entry point is called without per-argument conversion.
-    """
-    N = y.shape[1]
-    if slices is None and _use_long(x, plan, cache, N, stream):
-        _long_launch(x, [y], cache, [module_name], plan, epilogue, stream)
-        return
-    c32 = _native.c32
-    rc = _native.raw("pl_lora_fused")(
-        c32(_native.dtype_code(x.dtype)), ctypes.c_void_p(x.data_ptr()), ctypes.c_int64(x.stride(0)),
-        c32(x.shape[1]), ctypes.c_void_p(y.data_ptr()), ctypes.c_int64(y.stride(0)), c32(N),
-        *_cache_args_c(cache, module_name), *plan.launch_args_c,
-        c32(choose_slices(plan, N) if slices is None else slices), c32(epilogue), ctypes.c_void_p(stream))
+    """pl_lora_fused on operands the caller has checked, or the two-launch path where long_ok prefers it."""
+    K, N = x.shape[1], y.shape[1]
+    if slices is None:
+        if _use_long(x, plan, cache, N, stream):
+            _long_launch(x, [y], cache, [module_name], plan, epilogue, stream)
+            return
+        slices = choose_slices(plan, N)
+    rc = _native.calls().pl_lora_fused(
+        _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), K, y.data_ptr(), y.stride(0), N,
+        *_cache_args(cache, module_name), *plan.launch_args, slices, epilogue, stream)
     if rc:
         _native.check(rc, "pl_lora_fused")
 
@@ -694,20 +634,15 @@ def lora_fused_stacked(
     if slices is None and _use_long(x, plan, cache, sum(y.shape[1] for y in ys), stream):
         _long_launch(x, ys, cache, module_names, plan, epilogue, _stream(x.device))
         return ys
-    specs, mods, (yp, ldy, nn_) = _fused_set(cache, module_names)
-    for i, y in enumerate(ys):
-        yp[i] = y.data_ptr()
-        ldy[i] = y.stride(0)
-    n_slices = slices if slices is not None else choose_slices(plan, min(spec.out_features for spec in specs))
+    _, mods, widths, _ = _module_set(cache, module_names)
     arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
-    _native.check(
-        _native.load().pl_lora_fused_stacked(
-            _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], len(ys), mods, yp, ldy, nn_,
-            arena, table, n_mod, ldt, *plan.launch_args, n_slices, epilogue,
-            _stream(x.device) if stream is None else stream,
-        ),
-        "pl_lora_fused_stacked",
-    )
+    rc = _native.calls().pl_lora_fused_stacked(
+        _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], len(ys), mods,
+        tuple([y.data_ptr() for y in ys]), tuple([y.stride(0) for y in ys]), widths, arena, table, n_mod, ldt,
+        *plan.launch_args, choose_slices(plan, min(widths)) if slices is None else slices, epilogue,
+        _stream(x.device) if stream is None else stream)
+    if rc:
+        _native.check(rc, "pl_lora_fused_stacked")
     return ys
 
 
@@ -721,7 +656,7 @@ def _check_stacked(x: torch.Tensor, ys: list, cache, module_names: list, plan: S
     _check_operands(x, ys[0], cache, module_names[0], plan.tokens_cap)
     if not _tiled_ok(x, ys[0]):
         raise ValueError("lora_fused needs 16-byte aligned rows and K, N multiples of 16 bytes")
-    specs, _ = _module_set(cache, module_names)
+    specs = _module_set(cache, module_names)[0]
     chunk = 16 // x.element_size()
     for y, spec in zip(ys[1:], specs[1:]):
         if spec.in_features != x.shape[1]:
@@ -766,26 +701,20 @@ def lora_expand_stacked(results: list, ys: list, cache, module_names: list, *,
             raise TypeError(f"y {y.dtype} on {y.device} must match the adapter cache ({cache.dtype} on {cache.device})")
         if not res.valid:
             raise RuntimeError("the shrink result was overwritten by a later shrink on the same workspace")
-    lib = _native.load()
     r0 = results[0]
     batch = r0.batch
     if batch is not None and batch.n == n and all(r.batch is batch and r.index == i for i, r in enumerate(results)):
-        ws = batch.ptrs  # the shrink's own pointer array, in the same order
+        ws = batch.ptrs  # the shrink's own addresses, in the same order
     else:
-        ws = (ctypes.c_void_p * n)(*(r.buf.data_ptr() for r in results))
-    _, mods = _module_set(cache, module_names)
-    yp = (ctypes.c_void_p * n)(*(y.data_ptr() for y in ys))
-    ldy = (ctypes.c_int64 * n)(*(y.stride(0) for y in ys))
-    nn_ = (ctypes.c_int32 * n)(*(int(y.shape[1]) for y in ys))
-    _native.check(
-        lib.pl_sgmv_expand_stacked(
-            _native.dtype_code(ys[0].dtype), ws, r0.ldt, r0.rows, r0.planes, cache.arena.data_ptr(),
-            cache.table.data_ptr(), len(cache.module_index), n, mods, plan.tok.data_ptr(), plan.groups.data_ptr(),
-            plan.meta.data_ptr(), max(1, plan.group_cap), plan.group_tokens, yp, ldy, nn_, epilogue,
-            _stream(ys[0].device) if stream is None else stream,
-        ),
-        "pl_sgmv_expand_stacked",
-    )
+        ws = tuple([r.buf.data_ptr() for r in results])
+    arena, table, n_mod, _, _ = _cache_args(cache, module_names[0])
+    rc = _native.calls().pl_sgmv_expand_stacked(
+        _native.dtype_code(ys[0].dtype), ws, r0.ldt, r0.rows, r0.planes, arena,
+        table, n_mod, n, _module_set(cache, module_names)[1], *plan.launch_args, tuple([y.data_ptr() for y in ys]),
+        tuple([y.stride(0) for y in ys]), tuple([y.shape[1] for y in ys]), epilogue,
+        _stream(ys[0].device) if stream is None else stream)
+    if rc:
+        _native.check(rc, "pl_sgmv_expand_stacked")
     return ys
 
 
@@ -879,45 +808,47 @@ def lora_decode_stacked(x: torch.Tensor, ys: list, cache, module_names: list, pl
         raise ValueError(f"a decode launch serves 1..{_native.PL_MAX_STACKED_MODULES} modules with one y each")
     if not decode_ok(plan):
         raise ValueError("lora_decode_stacked takes plans of 16-token groups")
-    specs, mods, arrays = _fused_set(cache, module_names)
-    K = int(x.shape[1]) if x.dim() == 2 else -1
-    if x.dim() != 2 or x.shape[0] != plan.tokens_cap or any(sp.in_features != K for sp in specs):
-        raise ValueError(f"x must be [{plan.tokens_cap}, in_features] for every module, got {list(x.shape)}")
-    if x.dtype != cache.dtype or x.device != cache.device:
-        raise TypeError(f"x {x.dtype} on {x.device} must match the adapter cache ({cache.dtype} on {cache.device})")
-    for y, spec in zip(ys, specs):
+    _, mods, widths, fin = _module_set(cache, module_names)
+    tokens, dtype, device = plan.tokens_cap, cache.dtype, cache.device
+    K = x.shape[1] if x.dim() == 2 else -1
+    if K < 0 or x.shape[0] != tokens or K != fin:
+        raise ValueError(f"x must be [{tokens}, in_features] for every module, got {list(x.shape)}")
+    if x.dtype != dtype or x.device != device:
+        raise TypeError(f"x {x.dtype} on {x.device} must match the adapter cache ({dtype} on {device})")
+    for y, N, name in zip(ys, widths, module_names):
         _require_gpu(y, "lora_decode_stacked")
-        if y.dim() != 2 or y.shape[0] != plan.tokens_cap or y.shape[1] != spec.out_features:
-            raise ValueError(f"y of {spec.name!r} must be [{plan.tokens_cap}, {spec.out_features}], got {list(y.shape)}")
-        if y.dtype != cache.dtype or y.device != cache.device:
-            raise TypeError(f"y {y.dtype} on {y.device} must match the adapter cache ({cache.dtype} on {cache.device})")
-    lib = _native.load()
-    dt = _native.dtype_code(x.dtype)
+        if y.shape != (tokens, N):
+            raise ValueError(f"y of {name!r} must be [{tokens}, {N}], got {list(y.shape)}")
+        if y.dtype != dtype or y.device != device:
+            raise TypeError(f"y {y.dtype} on {y.device} must match the adapter cache ({dtype} on {device})")
+    dt = _native.dtype_code(dtype)
     ldt = -(-cache.rank8_cap // 32) * 32  # plane rows of whole 128-byte lines
     if stream is None:
-        stream = _stream(x.device)
-    rows = max(1, plan.tokens_cap)
-    splits, planes, nbytes = _shrink_geometry(lib, dt, K, x.dtype, plan, rows, ldt, k_splits)
-    wss, bufs, ptrs = _workspace_set(x.device, stream, n, nbytes)
+        stream = _stream(device)
+    rows = max(1, tokens)
+    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, dtype, plan, rows, ldt, k_splits)
+    wss, _, ptrs, size = _workspace_set(device, stream, n, nbytes)
     for ws in wss:
         ws.owner = None  # any earlier shrink's planes there are overwritten by this launch
-    cap = max(1, plan.group_cap)
-    need = int(lib.pl_decode_counter_ints(cap, n))
-    counters = handoff_counters(x.device, stream).get(need)
-    yp, ldy, nn_ = arrays
-    for i, y in enumerate(ys):
-        yp[i] = y.data_ptr()
-        ldy[i] = y.stride(0)
-    _native.check(
-        lib.pl_lora_decode_stacked(
-            dt, x.data_ptr(), x.stride(0), K, cache.arena.data_ptr(), cache.table.data_ptr(), len(cache.module_index),
-            n, mods, ptrs, plan.tok.data_ptr(), plan.groups.data_ptr(), plan.meta.data_ptr(), cap, plan.group_tokens,
-            min(b.numel() for b in bufs), ldt, rows, splits, yp, ldy, nn_, epilogue, counters.data_ptr(),
-            counters.numel(), DECODE_SPIN_LIMIT, stream,
-        ),
-        "pl_lora_decode_stacked",
-    )
+    counters = handoff_counters(device, stream).get(_counter_ints(plan.launch_args[3], n))
+    arena, table, n_mod, _, _ = _cache_args(cache, module_names[0])
+    rc = _native.calls().pl_lora_decode_stacked(
+        dt, x.data_ptr(), x.stride(0), K, arena, table, n_mod, n, mods, ptrs, *plan.launch_args, size, ldt, rows,
+        splits, tuple([y.data_ptr() for y in ys]), tuple([y.stride(0) for y in ys]), widths, epilogue,
+        counters.data_ptr(), counters.numel(), DECODE_SPIN_LIMIT, stream)
+    if rc:
+        _native.check(rc, "pl_lora_decode_stacked")
     return ys
+
+
+_COUNTER_INTS: dict[tuple[int, int], int] = {}
+
+
+def _counter_ints(group_cap: int, n: int) -> int:
+    got = _COUNTER_INTS.get((group_cap, n))
+    if got is None:
+        got = _COUNTER_INTS[group_cap, n] = int(_native.load().pl_decode_counter_ints(group_cap, n))
+    return got
 
 
 def lora_apply_rows(
@@ -936,7 +867,6 @@ def lora_apply_rows(
     _check_operands(x, y, cache, module_name, int(row_slot.numel()) * int(row_len))
     if int(seq_lens.numel()) != int(row_slot.numel()):
         raise ValueError("row_slot and seq_lens must have the same length")
-    lib = _native.load()
     if x.stride(-1) != 1:
         x = x.contiguous()
     y_work = y if y.stride(-1) == 1 else y.contiguous()
@@ -946,31 +876,13 @@ def lora_apply_rows(
     tmp = torch.empty(max(1, T * ldt), dtype=torch.float32, device=x.device)
     row_slot = _i32(row_slot)
     seq_lens = _i32(seq_lens)
-    _native.check(
-        lib.pl_lora_apply_rows(
-            _native.dtype_code(x.dtype),
-            x.data_ptr(),
-            x.stride(0),
-            int(x.shape[1]),
-            y_work.data_ptr(),
-            y_work.stride(0),
-            int(y_work.shape[1]),
-            cache.arena.data_ptr(),
-            cache.table.data_ptr(),
-            cache.num_slots,
-            len(cache.module_index),
-            cache.module_index[module_name],
-            row_slot.data_ptr(),
-            seq_lens.data_ptr(),
-            rows,
-            int(row_len),
-            tmp.data_ptr(),
-            ldt,
-            epilogue,
-            _stream(x.device),
-        ),
-        "pl_lora_apply_rows",
-    )
+    arena, table, n_mod, column, _ = _cache_args(cache, module_name)
+    rc = _native.calls().pl_lora_apply_rows(
+        _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], y_work.data_ptr(), y_work.stride(0),
+        y_work.shape[1], arena, table, cache.num_slots, n_mod, column, row_slot.data_ptr(), seq_lens.data_ptr(), rows,
+        int(row_len), tmp.data_ptr(), ldt, epilogue, _stream(x.device))
+    if rc:
+        _native.check(rc, "pl_lora_apply_rows")
     if y_work is not y:
         y.copy_(y_work)
     return y
@@ -1082,7 +994,7 @@ def sgmv_lora_a_fwd(
     if parts is None:
         _native.check(lib.pl_sgmv_lora_a_ref(*head, 0, 0, stream), "pl_sgmv_lora_a_ref")
     else:
-        _native.check(lib.pl_sgmv_lora_a_ref_parts(*head, *parts[0], stream), "pl_sgmv_lora_a_ref_parts")
+        _native.check(_native.calls().pl_sgmv_lora_a_ref_parts(*head, *parts[0], stream), "pl_sgmv_lora_a_ref_parts")
     return output
 
 
@@ -1130,7 +1042,7 @@ def sgmv_lora_b_fwd(
     if parts is None:
         _native.check(lib.pl_sgmv_lora_b_ref(*head, 0, 0, stream), "pl_sgmv_lora_b_ref")
     else:
-        _native.check(lib.pl_sgmv_lora_b_ref_parts(*head, *parts[0], stream), "pl_sgmv_lora_b_ref_parts")
+        _native.check(_native.calls().pl_sgmv_lora_b_ref_parts(*head, *parts[0], stream), "pl_sgmv_lora_b_ref_parts")
     if work is not output:
         output.copy_(work)
     return output
