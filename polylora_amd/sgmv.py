@@ -178,14 +178,27 @@ def _workspace(device: torch.device, stream: int, position: int = 0) -> _Workspa
 # splits: the expand holds one register set per split, and with 9..16 it runs
 # half as many waves per SIMD (decode down_proj, K = 14336: 14 splits 22.7 us
 # for the pair, 8 splits 21.9 us).
+# Small launches wait for one workgroup's chain of K steps instead: with few
+# groups, splits of 256 up to 4 of them (one decode launch, rank 64, 40 rows:
+# K = 1024 8.0 -> 6.0 us, K = 2048 9.5 -> 8.2; 256 rows over 64 adapters 9.0 ->
+# 7.0 and 15.0 -> 14.3), and with at most 16 groups splits of 512 up to 16
+# (8 rows, rank 64: K = 4096 8.6 -> 8.1, q/k/v 9.2 -> 8.9, K = 14336 12.1 -> 11.4;
+# at 24 groups and three modules it no longer pays: 8.9 -> 9.0).
 _K_PER_SPLIT = 1024
 _TARGET_SHRINK_BLOCKS = 2048
 _MAX_K_SPLITS = 8
+_FEW_GROUPS = 128
+_FEWEST_GROUPS = 16
 
 
 def choose_k_splits(group_cap: int, K: int, dtype: torch.dtype) -> int:
-    """K splits of the shrink: about one per 1024 of K (at most 8), fewer when the group count alone fills the GPU."""
+    """K splits of the shrink: about one per 1024 of K (at most 8), more for few groups, fewer when the group count
+    alone fills the GPU."""
     by_k = min(_MAX_K_SPLITS, max(1, -(-K // _K_PER_SPLIT)))
+    if group_cap <= _FEWEST_GROUPS:
+        by_k = max(by_k, min(2 * _MAX_K_SPLITS, K // 512))
+    if group_cap <= _FEW_GROUPS:
+        by_k = max(by_k, min(4, K // 256))
     by_groups = max(1, -(-_TARGET_SHRINK_BLOCKS // max(1, group_cap)))
     return min(by_k, by_groups)
 
@@ -238,8 +251,9 @@ def lora_apply(
     x: [rows*row_len, in_features], y: [rows*row_len, out_features], both of
     the cache's dtype, on the cache's device.  Long adapter segments go to
     the fused kernel (lora_fused) or, with more data or ranks above its
-    limit, to the two-launch path (long_ok), unless k_splits asks for the
-    split pair;
+    limit, to the two-launch path (long_ok); other plans of 16-token groups
+    to the one-launch decode kernel (lora_decode_stacked) where it is not
+    slower; all unless k_splits asks for the split pair;
     x / y that do not meet the tiled path's alignment go to the row-based HIP
     kernels.
     """
@@ -254,6 +268,9 @@ def lora_apply(
             return y
         if long_ok(plan, cache, x.shape[1], y.shape[1]):
             _long_launch(x, [y], cache, [module_name], plan, epilogue, _stream(x.device))
+            return y
+        if _one_launch_ok(plan, cache, x.shape[1], y.shape[1]):
+            _decode_launch(x, [y], cache, [module_name], plan, None, epilogue, _stream(x.device))
             return y
     dt = _native.dtype_code(x.dtype)
     K = x.shape[1]
@@ -808,7 +825,7 @@ def lora_decode_stacked(x: torch.Tensor, ys: list, cache, module_names: list, pl
         raise ValueError(f"a decode launch serves 1..{_native.PL_MAX_STACKED_MODULES} modules with one y each")
     if not decode_ok(plan):
         raise ValueError("lora_decode_stacked takes plans of 16-token groups")
-    _, mods, widths, fin = _module_set(cache, module_names)
+    _, _, widths, fin = _module_set(cache, module_names)
     tokens, dtype, device = plan.tokens_cap, cache.dtype, cache.device
     K = x.shape[1] if x.dim() == 2 else -1
     if K < 0 or x.shape[0] != tokens or K != fin:
@@ -821,11 +838,30 @@ def lora_decode_stacked(x: torch.Tensor, ys: list, cache, module_names: list, pl
             raise ValueError(f"y of {name!r} must be [{tokens}, {N}], got {list(y.shape)}")
         if y.dtype != dtype or y.device != device:
             raise TypeError(f"y {y.dtype} on {y.device} must match the adapter cache ({dtype} on {device})")
+    _decode_launch(x, ys, cache, module_names, plan, k_splits, epilogue, _stream(device) if stream is None else stream)
+    return ys
+
+
+def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -> bool:
+    """Whether lora_apply runs one pl_lora_decode_stacked launch instead of the split pair.
+
+    One launch saves the second one's host time (10.4 -> 7.3 us a call where
+    the GPU needs less) and is about even on the GPU, except above rank 64,
+    whose shrink passes all arrive on one counter (37 rows, 14336 -> 4096, rank
+    128: 13.8 -> 15.4 us), and for many rows of wide outputs (256 rows, 4096 ->
+    14336, rank 64: 18.6 -> 19.5 us).
+    """
+    return (plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
+            and (plan.tokens_cap < 256 or out_features <= 2 * in_features))
+
+
+def _decode_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, k_splits, epilogue: int, stream: int) -> None:
+    """pl_lora_decode_stacked on operands the caller has checked."""
+    n, device, dtype = len(ys), cache.device, cache.dtype
+    _, mods, widths, K = _module_set(cache, module_names)
     dt = _native.dtype_code(dtype)
     ldt = -(-cache.rank8_cap // 32) * 32  # plane rows of whole 128-byte lines
-    if stream is None:
-        stream = _stream(device)
-    rows = max(1, tokens)
+    rows = max(1, plan.tokens_cap)
     splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, dtype, plan, rows, ldt, k_splits)
     wss, _, ptrs, size = _workspace_set(device, stream, n, nbytes)
     for ws in wss:
@@ -838,7 +874,6 @@ def lora_decode_stacked(x: torch.Tensor, ys: list, cache, module_names: list, pl
         counters.data_ptr(), counters.numel(), DECODE_SPIN_LIMIT, stream)
     if rc:
         _native.check(rc, "pl_lora_decode_stacked")
-    return ys
 
 
 _COUNTER_INTS: dict[tuple[int, int], int] = {}

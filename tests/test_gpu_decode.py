@@ -226,3 +226,30 @@ def test_decode_launch_rejects_long_group_plans(gpu):
     x = torch.zeros(400, 256, dtype=torch.bfloat16, device=gpu)
     with pytest.raises(ValueError, match="16-token groups"):
         sgmv.lora_decode_stacked(x, [torch.zeros_like(x)], cache, ["m"], plan)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rows,row_len,K,N,rank,one", [
+    (1, 1, 1024, 1024, 16, True), (7, 3, 520, 2056, 64, True), (7, 3, 520, 1040, 64, True), (40, 1, 2048, 264, 40, True),
+    (300, 1, 264, 520, 8, True), (300, 1, 264, 536, 8, False), (5, 1, 264, 264, 72, False)])
+def test_lora_apply_in_one_launch_equals_the_split_pair(gpu, monkeypatch, dtype, rows, row_len, K, N, rank, one):
+    """lora_apply on plans of 16-token groups: one launch by its rule (rank up to 64; below 256 tokens or N up to
+    2 K), bit for bit the split pair at the same K splits, also for strided rows of x and y."""
+    launches = []
+    launch = sgmv._decode_launch
+    monkeypatch.setattr(sgmv, "_decode_launch", lambda *a: (launches.append(1), launch(*a))[1])
+    g = torch.Generator().manual_seed(rows + K + N)
+    adapters = {f"a{i}": {"m": peft_layer(g, K, N, max(1, rank >> i), 2.0)} for i in range(3)}
+    cache = make_cache(adapters, {"m": (K, N)}, 3, rank, gpu, dtype)
+    ids = [["a0", "a1", "a2", "__base__"][i] for i in torch.randint(0, 4, (rows,), generator=g).tolist()]
+    seq = torch.randint(0, row_len + 1, (rows,), generator=g, dtype=torch.int32).to(gpu)
+    plan = sgmv.SgmvPlan(cache.ensure_resident(ids), seq, row_len, cache.num_slots, distinct_slots=3)
+    wide_x = torch.randn(rows * row_len, K + 16, generator=g).to(dtype).to(gpu)
+    wide_y = torch.randn(rows * row_len, N + 32, generator=g).to(dtype).to(gpu)
+    want, got = wide_y.clone(), wide_y.clone()
+    x = wide_x[:, 16:]
+    sgmv.lora_apply(x, want[:, :N], cache, "m", plan, k_splits=sgmv.choose_k_splits(plan.group_cap, K, dtype))
+    assert not launches
+    sgmv.lora_apply(x, got[:, :N], cache, "m", plan)
+    assert torch.equal(got, want) and bool(launches) == one
+    assert not sgmv.decode_waits_timed_out(gpu)
