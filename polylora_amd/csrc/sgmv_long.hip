@@ -271,7 +271,7 @@ __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int jo
 }
 
 template <int DT, int JT, int RT, bool XNT>
-__global__ __launch_bounds__(64 * kLWaves) void pl_long_shrink(pl_long_args a) {
+__global__ __launch_bounds__(64 * kLWaves, RT * JT <= 4 ? 3 : 2) void pl_long_shrink(pl_long_args a) {
   __shared__ __attribute__((aligned(16))) char smem[pl_long_shrink_lds<DT, JT, RT>()];
   const int xcd = (int)(blockIdx.x % kXcds);
   int rest = (int)(blockIdx.x / kXcds);
@@ -325,18 +325,20 @@ __global__ __launch_bounds__(64 * kLWaves) void pl_long_shrink(pl_long_args a) {
 
 // ------------------------------------------------------------------ expand
 
-template <int DT>
+// Above two rank steps a wave owns half the columns, so that its B fits the
+// registers of three workgroups per CU (rank 256, 5915 tokens, 4096 columns:
+// 51 -> 40 us; rank 128, 4138 tokens: 24.7 -> 23.1 us).
+template <int DT, int RSMAX>
 struct pl_long_shape {
   typedef typename pl_traits<DT>::T T;
-  enum { kCols = kLRowBytes / (int)sizeof(T) };  // columns per wave
+  enum { kCols = (RSMAX > 2 ? kLRowBytes / 2 : kLRowBytes) / (int)sizeof(T) };  // columns per wave
   enum { kChunk = kLWaves * kCols };       // columns per workgroup
   enum { kPad = 16 / (int)sizeof(T) };
   enum { kDRow = kCols + kPad };
 };
 
-// RS: rank steps of one MFMA wave load held in registers; CT: 16-column
-// tiles held at a time (a wave's columns are taken CT tiles after another).
-template <int DT, int RS, int CT, int kTRow>
+// One run of tiles of one slot; RS: rank steps of one MFMA wave load.
+template <int DT, int RS, int RSMAX, int kTRow>
 __device__ __forceinline__ void pl_long_expand_run(const pl_long_args& a, int job, int chunk,
                                                    const pl_slot_entry& e, int n_tiles,
                                                    const int (&tlen)[kLUnitMax],
@@ -346,11 +348,11 @@ __device__ __forceinline__ void pl_long_expand_run(const pl_long_args& a, int jo
   typedef typename pl_traits<DT>::T T;
   typedef typename pl_traits<DT>::T4 T4;
   typedef typename pl_traits<DT>::T8 T8;
-  typedef pl_long_shape<DT> S;
+  typedef pl_long_shape<DT, RSMAX> S;
   constexpr int E = pl_traits<DT>::E;
   constexpr int kRStep = 4 * E;
-  constexpr int kW = CT * 16;                            // columns held at a time
-  constexpr int kYLanes = kW * (int)sizeof(T) / 16;      // lanes per y row
+  constexpr int CT = S::kCols / 16;                          // 16-column MFMA tiles per wave
+  constexpr int kYLanes = S::kCols * (int)sizeof(T) / 16;    // lanes per y row
   constexpr int kYRows = 64 / kYLanes;
   constexpr int kYLoads = 16 / kYRows;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -367,98 +369,95 @@ __device__ __forceinline__ void pl_long_expand_run(const pl_long_args& a, int jo
   const int yq = lane % kYLanes;
   const int yr0 = lane / kYLanes;
 
-  for (int h = 0; h < S::kCols / kW; ++h) {
-    const int cb = chunk * S::kChunk + wave * S::kCols + h * kW;
-    if (cb >= N) return;
-    const bool cok = cb + yq * E < N;
-    auto load = [&](pl_u32x4 (&yv)[kYLoads], int i) {
-      const bool on = i < n_tiles;
-      const int len = on ? tlen[i] : 0;
+  const int cb = chunk * S::kChunk + wave * S::kCols;
+  if (cb >= N) return;
+  const bool cok = cb + yq * E < N;
+  auto load = [&](pl_u32x4 (&yv)[kYLoads], int i) {
+    const bool on = i < n_tiles;
+    const int len = on ? tlen[i] : 0;
 #pragma unroll
-      for (int q = 0; q < kYLoads; ++q) {
-        const int r = yr0 + kYRows * q;
-        yv[q] = pl_ld16_nt_or0(y + (int64_t)ltok[(on ? i : 0) * 16 + r] * ldy + cb + yq * E, r < len && cok);
-      }
-    };
-    pl_u32x4 ya[kYLoads], yb[kYLoads];
-    load(ya, 0);
-    pl_u32x4 bf[RS][CT];
-#pragma unroll
-    for (int s = 0; s < RS; ++s) {
-      // B's MFMA blocks: the 16-column tile at nb (nt columns), rank block
-      // j0 (wb wide) starts at nb*r8 + j0*nt
-      const int j0 = s * kRStep;
-      const int wb = min(kRStep, r8 - j0);
-#pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        const int nb = cb + ct * 16;
-        const int nt = min(16, N - nb);
-        bf[s][ct] = pl_ld16_or0(Bc + (int64_t)nb * r8 + (int64_t)j0 * nt + li * wb + lg * E,
-                                li < nt && j0 + lg * E < r8);
-      }
+    for (int q = 0; q < kYLoads; ++q) {
+      const int r = yr0 + kYRows * q;
+      yv[q] = pl_ld16_nt_or0(y + (int64_t)ltok[(on ? i : 0) * 16 + r] * ldy + cb + yq * E, r < len && cok);
     }
-    auto apply = [&](const pl_u32x4 (&yv)[kYLoads], int i) {
-      pl_u32x4 tf[RS];
+  };
+  pl_u32x4 ya[kYLoads], yb[kYLoads];
+  load(ya, 0);
+  pl_u32x4 bf[RS][CT];
 #pragma unroll
-      for (int s = 0; s < RS; ++s)
-        tf[s] = *reinterpret_cast<const pl_u32x4*>(lt + (i * 16 + li) * kTRow + s * kRStep + lg * E);
-      pl_f32x4 d[CT];
+  for (int s = 0; s < RS; ++s) {
+    // B's MFMA blocks: the 16-column tile at nb (nt columns), rank block
+    // j0 (wb wide) starts at nb*r8 + j0*nt
+    const int j0 = s * kRStep;
+    const int wb = min(kRStep, r8 - j0);
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) d[ct] = pl_f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int ct = 0; ct < CT; ++ct) {
+      const int nb = cb + ct * 16;
+      const int nt = min(16, N - nb);
+      bf[s][ct] = pl_ld16_or0(Bc + (int64_t)nb * r8 + (int64_t)j0 * nt + li * wb + lg * E,
+                              li < nt && j0 + lg * E < r8);
+    }
+  }
+  auto apply = [&](const pl_u32x4 (&yv)[kYLoads], int i) {
+    pl_u32x4 tf[RS];
 #pragma unroll
-      for (int s = 0; s < RS; ++s)
+    for (int s = 0; s < RS; ++s)
+      tf[s] = *reinterpret_cast<const pl_u32x4*>(lt + (i * 16 + li) * kTRow + s * kRStep + lg * E);
+    pl_f32x4 d[CT];
 #pragma unroll
-        for (int ct = 0; ct < CT; ++ct) d[ct] = pl_mfma_chunk<DT>(bf[s][ct], tf[s], d[ct]);
-      // d[ct][v] = delta(column cb + ct*16 + 4*lg + v, token li): scale and round,
-      // then through this wave's LDS tile to the row-major layout of y
+    for (int ct = 0; ct < CT; ++ct) d[ct] = pl_f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int ct = 0; ct < CT; ++ct) {
-        T4 dd;
+    for (int s = 0; s < RS; ++s)
 #pragma unroll
-        for (int v = 0; v < 4; ++v) dd[v] = (T)pl_delta<DT>(d[ct][v], scale, scale_t, a.epilogue);
-        *reinterpret_cast<T4*>(dw + li * S::kDRow + ct * 16 + lg * 4) = dd;
-      }
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-      const int len = tlen[i];
+      for (int ct = 0; ct < CT; ++ct) d[ct] = pl_mfma_chunk<DT>(bf[s][ct], tf[s], d[ct]);
+    // d[ct][v] = delta(column cb + ct*16 + 4*lg + v, token li): scale and round,
+    // then through this wave's LDS tile to the row-major layout of y
 #pragma unroll
-      for (int q = 0; q < kYLoads; ++q) {
-        const int r = yr0 + kYRows * q;
-        const pl_u32x4 dv = *reinterpret_cast<const pl_u32x4*>(dw + r * S::kDRow + yq * E);
-        if (r < len && cok) {
-          pl_u32x4 out;
-          if constexpr (E == 8) {
-            T8 yy = __builtin_bit_cast(T8, yv[q]);
-            const T8 dd = __builtin_bit_cast(T8, dv);
+    for (int ct = 0; ct < CT; ++ct) {
+      T4 dd;
 #pragma unroll
-            for (int c = 0; c < 8; ++c) yy[c] = (T)((float)yy[c] + (float)dd[c]);
-            out = __builtin_bit_cast(pl_u32x4, yy);
-          } else {
-            out = __builtin_bit_cast(pl_u32x4, __builtin_bit_cast(pl_f32x4, yv[q]) +
-                                                   __builtin_bit_cast(pl_f32x4, dv));
-          }
-          pl_st16_nt(y + (int64_t)ltok[i * 16 + r] * ldy + cb + yq * E, out);
+      for (int v = 0; v < 4; ++v) dd[v] = (T)pl_delta<DT>(d[ct][v], scale, scale_t, a.epilogue);
+      *reinterpret_cast<T4*>(dw + li * S::kDRow + ct * 16 + lg * 4) = dd;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+    const int len = tlen[i];
+#pragma unroll
+    for (int q = 0; q < kYLoads; ++q) {
+      const int r = yr0 + kYRows * q;
+      const pl_u32x4 dv = *reinterpret_cast<const pl_u32x4*>(dw + r * S::kDRow + yq * E);
+      if (r < len && cok) {
+        pl_u32x4 out;
+        if constexpr (E == 8) {
+          T8 yy = __builtin_bit_cast(T8, yv[q]);
+          const T8 dd = __builtin_bit_cast(T8, dv);
+#pragma unroll
+          for (int c = 0; c < 8; ++c) yy[c] = (T)((float)yy[c] + (float)dd[c]);
+          out = __builtin_bit_cast(pl_u32x4, yy);
+        } else {
+          out = __builtin_bit_cast(pl_u32x4, __builtin_bit_cast(pl_f32x4, yv[q]) +
+                                                 __builtin_bit_cast(pl_f32x4, dv));
         }
+        pl_st16_nt(y + (int64_t)ltok[i * 16 + r] * ldy + cb + yq * E, out);
       }
-      // the next tile rewrites the LDS tile only after these reads (in-order LDS)
-      __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
-    };
-    for (int i = 0; i < n_tiles; i += 2) {
-      load(yb, i + 1);
-      __builtin_amdgcn_sched_barrier(0);
-      apply(ya, i);
-      if (i + 1 >= n_tiles) break;
-      load(ya, i + 2);
-      __builtin_amdgcn_sched_barrier(0);
-      apply(yb, i + 1);
     }
+    // the next tile rewrites the LDS tile only after these reads (in-order LDS)
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  };
+  for (int i = 0; i < n_tiles; i += 2) {
+    load(yb, i + 1);
+    __builtin_amdgcn_sched_barrier(0);
+    apply(ya, i);
+    if (i + 1 >= n_tiles) break;
+    load(ya, i + 2);
+    __builtin_amdgcn_sched_barrier(0);
+    apply(yb, i + 1);
   }
 }
 
 template <int DT, int RSMAX, int NT>
-__global__ __launch_bounds__(64 * kLWaves) void pl_long_expand(pl_long_args a) {
+__global__ __launch_bounds__(64 * kLWaves, RSMAX <= 4 ? 3 : 2) void pl_long_expand(pl_long_args a) {
   typedef typename pl_traits<DT>::T T;
-  typedef pl_long_shape<DT> S;
-  constexpr int kCT = S::kCols / 16;
+  typedef pl_long_shape<DT, RSMAX> S;
   __shared__ __attribute__((aligned(16))) T delta[kLWaves][16 * S::kDRow];
   constexpr int kTRow = RSMAX * 4 * pl_traits<DT>::E + S::kPad;
   __shared__ __attribute__((aligned(16))) T lt[NT * 16 * kTRow];
@@ -551,13 +550,13 @@ __global__ __launch_bounds__(64 * kLWaves) void pl_long_expand(pl_long_args a) {
       if (e.rank > 0) {
         const int r = (e.rank8 + 4 * pl_traits<DT>::E - 1) / (4 * pl_traits<DT>::E);
         if (RSMAX == 1 || r == 1)
-          pl_long_expand_run<DT, 1, kCT, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
+          pl_long_expand_run<DT, 1, RSMAX, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
         else if (RSMAX == 2 || r == 2)
-          pl_long_expand_run<DT, 2 < RSMAX ? 2 : RSMAX, kCT, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
+          pl_long_expand_run<DT, 2 < RSMAX ? 2 : RSMAX, RSMAX, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
         else if (RSMAX == 4 || r <= 4)
-          pl_long_expand_run<DT, 4 < RSMAX ? 4 : RSMAX, kCT, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
+          pl_long_expand_run<DT, 4 < RSMAX ? 4 : RSMAX, RSMAX, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
         else
-          pl_long_expand_run<DT, RSMAX, 4, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
+          pl_long_expand_run<DT, RSMAX, RSMAX, kTRow>(a, job, chunk, e, n, rl, lk, lti, dw);
       }
     }
     i0 += n;
@@ -668,8 +667,8 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
     pl_set_error("group capacity %lld out of range", (long long)group_cap);
     return PL_ERR_LIMIT;
   }
-  const int chunk = dtype == PL_F32 ? (int)pl_long_shape<PL_F32>::kChunk
-                                    : (int)pl_long_shape<PL_BF16>::kChunk;
+  const int rs = (ldt + 4 * E - 1) / (4 * E);  // rank steps of the expand
+  const int chunk = kLWaves * (rs > 2 ? kLRowBytes / 2 : kLRowBytes) / es;  // columns per expand workgroup
   pl_long_args a;
   int64_t n_chunks = 0;
   for (int j = 0; j < n_modules; ++j) {
