@@ -734,11 +734,17 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   a.n_chunks = (int32_t)n_chunks;
   a.ldt = long_ldt(ldt);
   // Shrink: two tiles per workgroup share each A load once the launch has
-  // 512 tiles (8192 tokens); below, one tile, for more workgroups (bf16,
-  // K = 4096, rank 64: 3023 tokens 31 against 40 us for the pair of launches,
-  // 5773 tokens 47 against 42 us).  Up to 64 ranks per pass.
-  const int rt = tiles >= 512 ? 2 : 1;
-  const int jt = ldt <= 16 ? 1 : ldt <= 32 ? 2 : 4;
+  // 512 tiles (8192 tokens), above rank 64 from 320 on; below, one tile, for
+  // more workgroups (bf16, K = 4096: rank 32 with 260 tiles 12 against 17 us, 520
+  // tiles 16 against 13; rank 64 with 354 tiles 17.4 against 17.0, fewer of them
+  // in use 13 against 18; rank 128 with 260 tiles 21 against 23, 354 tiles 24
+  // against 22).  Passes of 32 ranks balance better over the CUs than passes
+  // of 64 (rank 64, 520 tiles 16 against 18 us; K = 14336 44 against 56) until
+  // they make 1536 workgroups, when rereading x costs more (K = 14336, rank 128,
+  // 1040 tiles: 195 against 130 us).
+  const int rt = tiles >= (ldt > 64 ? 320 : 512) ? 2 : 1;
+  const int64_t blocks = tiles / rt * n_modules * ((ldt + 31) / 32);
+  const int jt = ldt <= 16 ? 1 : ldt <= 32 || blocks < 1536 ? 2 : 4;
   // Expand: tiles per workgroup, which share the workgroup's B: 4 above rank
   // 32 (2048 -> 8192, rank 64, 5773 tokens: 4 tiles 53, 2 tiles 60, 1 tile
   // 64 us), 2 below (4096 -> 2 x 14336, rank 32, 11557 tokens: 272, 270 and

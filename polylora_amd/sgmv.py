@@ -504,35 +504,49 @@ def fused_ok(plan: SgmvPlan, cache, in_features: int) -> bool:
     return plan.tokens_cap >= 64 * max(1, distinct) and plan.tokens_cap >= 1024
 
 
-# Ranks pl_lora_long_stacked takes (half of it in fp32), and the bytes of y
-# it must read and write to win over the fused launch: its second launch
-# costs about 5 us, which its faster streaming pays back from there on.
-# Measured on MI355X (bf16 unless said; y traffic of the plan's capacity,
-# fused against long): 2048 -> 8192 rank 16, 67 MB 16.4 / 19.3 us, 134 MB
-# 32.5 / 28.2; 4096 -> 4096 rank 32, 67 MB 21.0 / 23.3, 134 MB 40.9 / 35.5;
-# 4096 -> 2 x 14336 rank 16, 117 MB 28.4 / 26.3; fp32 768 -> 3072 rank 8,
-# 100 MB 20.6 / 22.5, 201 MB 37.4 / 35.4.  Above rank 64 the other choice is
-# the split pair, slower from 2048 tokens on (4096 -> 4096 rank 128, 1024
-# tokens 19.3 / 21.5 us, 2048 tokens 33.3 / 28.8).
-LONG_MAX_RANK = 256
+# Where pl_lora_long_stacked takes over from the fused launch.  Its second
+# launch costs about 5 us, which its faster streaming pays back
+# * up to rank 32, from LONG_MIN_Y_BYTES of y read and written on (y traffic of
+#   the plan's capacity, fused against long on MI355X, bf16 unless said: 2048 ->
+#   8192 rank 16, 67 MB 16.4 / 19.3 us, 134 MB 32.5 / 28.2; 4096 -> 4096 rank 32,
+#   67 MB 21.0 / 23.3, 134 MB 40.9 / 35.5; 4096 -> 2 x 14336 rank 16, 117 MB 28.4 /
+#   26.3; fp32 768 -> 3072 rank 8, 100 MB 20.6 / 22.5, 201 MB 37.4 / 35.4);
+# * above, where the fused launch rereads 64 ranks of A and B for every 16
+#   tokens, from LONG_MIN_BYTES of x and y on with rows of at least
+#   LONG_MIN_ROW_BYTES in all (rank 64: 4096 -> 4096, 2048 tokens 18.8 / 17.6 us,
+#   5600 tokens 29.3 / 26.5; 2048 -> 8192, 1024 tokens 16.2 / 17.3, 2560 tokens
+#   36.4 / 19.5; 14336 -> 4096, 2560 tokens 53.0 / 34.1; 1024 -> 1024, 5600 tokens
+#   10.0 / 12.1), twice that for several modules, which share a tile's x
+#   (2048 -> 2048, 512, 512, 65 MB 25.4 / 25.7).
+# Above rank 64 the other choice is the split pair, slower from
+# LONG_MIN_TOKENS on (4096 -> 4096 rank 128, 1024 tokens 19.3 / 21.5 us, 2048
+# tokens 33.3 / 28.8).
+LONG_MAX_RANK = 256  # half of it in fp32
 LONG_MIN_Y_BYTES = 112 << 20
+LONG_MIN_BYTES = 40 << 20
+LONG_MIN_ROW_BYTES = 8192
 LONG_MIN_TOKENS = 2048
 
 
-def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -> bool:
-    """Whether the two-launch path (pl_lora_long_stacked) suits a plan and modules of `out_features` columns in all."""
+def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules: int = 1) -> bool:
+    """Whether the two-launch path (pl_lora_long_stacked) suits a plan and `modules` of `out_features` columns in all."""
     distinct, rank, tokens = plan.distinct_slots, cache.rank8_cap, plan.tokens_cap
     if distinct is None or tokens < max(1024, 64 * max(1, distinct)):
         return False
     es = cache.dtype.itemsize
     if rank > FUSED_MAX_RANK:
         return rank <= LONG_MAX_RANK * 2 // max(2, es) and tokens >= LONG_MIN_TOKENS
-    return in_features <= FUSED_MAX_K and 2 * es * tokens * out_features >= LONG_MIN_Y_BYTES
+    if in_features > FUSED_MAX_K:
+        return False
+    if rank <= 32:
+        return 2 * es * tokens * out_features >= LONG_MIN_Y_BYTES
+    return (es * (in_features + out_features) >= LONG_MIN_ROW_BYTES
+            and es * tokens * (in_features + 2 * out_features) >= LONG_MIN_BYTES * min(modules, 2))
 
 
-def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, out_features: int, stream: int | None) -> bool:
+def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, out_features: int, stream: int | None, modules: int = 1) -> bool:
     """long_ok, on the current stream only: the workspace is allocated there."""
-    return long_ok(plan, cache, x.shape[1], out_features) and stream in (None, _stream(x.device))
+    return long_ok(plan, cache, x.shape[1], out_features, modules) and stream in (None, _stream(x.device))
 
 
 def _long_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, epilogue: int, stream: int) -> None:
@@ -648,7 +662,7 @@ def lora_fused_stacked(
     _check_stacked(x, ys, cache, module_names, plan)
     if cache.rank8_cap > FUSED_MAX_RANK:
         raise ValueError(f"lora_fused takes ranks up to {FUSED_MAX_RANK}; the cache holds up to {cache.rank8_cap}")
-    if slices is None and _use_long(x, plan, cache, sum(y.shape[1] for y in ys), stream):
+    if slices is None and _use_long(x, plan, cache, sum(y.shape[1] for y in ys), stream, len(ys)):
         _long_launch(x, ys, cache, module_names, plan, epilogue, _stream(x.device))
         return ys
     _, mods, widths, _ = _module_set(cache, module_names)

@@ -610,3 +610,20 @@ def test_long_workspace_size_is_64_bit():
     assert lib.pl_lora_long_workspace_bytes(_native.PL_F32, 3, 40) == 3 * 64 * 4  # rows of whole 32-rank blocks
     assert lib.pl_lora_long_workspace_bytes(_native.PL_BF16, 8, 264) == 0
     assert lib.pl_lora_long_workspace_bytes(_native.PL_F32, 8, 136) == 0
+
+
+@pytest.mark.parametrize("rank,tokens,fin,fout,modules,want", [
+    (16, 8192, 4096, 4096, 1, True), (16, 4096, 4096, 4096, 1, False), (32, 1024, 4096, 28672, 2, True),
+    (64, 2048, 4096, 4096, 1, True), (64, 1024, 4096, 4096, 1, False), (64, 16384, 1024, 1024, 1, False),
+    (64, 3980, 2048, 3072, 3, False), (64, 3980, 2048, 3072, 1, True), (64, 8192, 20480, 4096, 1, False),
+    (72, 2048, 64, 64, 1, True), (72, 2047, 64, 64, 1, False), (264, 4096, 64, 64, 1, False)])
+def test_long_path_rule(rank, tokens, fin, fout, modules, want):
+    """Which long-segment calls take the two-launch path (bf16, one adapter); never short segments."""
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    cache = Obj(rank8_cap=rank, dtype=torch.bfloat16)
+    assert sgmv.long_ok(Obj(distinct_slots=1, tokens_cap=tokens), cache, fin, fout, modules) == want
+    assert not sgmv.long_ok(Obj(distinct_slots=None, tokens_cap=tokens), cache, fin, fout, modules)
+    assert not sgmv.long_ok(Obj(distinct_slots=tokens // 32, tokens_cap=tokens), cache, fin, fout, modules)
