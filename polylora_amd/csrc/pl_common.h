@@ -165,6 +165,23 @@ __device__ __forceinline__ pl_f32x4 pl_mfma_chunk<PL_F32>(pl_u32x4 a, pl_u32x4 b
   return c;
 }
 
+// pl_mfma_chunk with short chains in fp32: the products of each word into a sum
+// of their own, those pairwise, and one addition to c, so that a wave's sum
+// over K is a chain of K / 16 additions instead of K.
+template <int DT>
+__device__ __forceinline__ pl_f32x4 pl_mfma_chunk_short(pl_u32x4 a, pl_u32x4 b, pl_f32x4 c) {
+  if constexpr (DT == PL_F32) {
+    pl_f32x4 p[4];
+#pragma unroll
+    for (int q = 0; q < 4; ++q)
+      p[q] = __builtin_amdgcn_mfma_f32_16x16x4f32(__uint_as_float(a[q]), __uint_as_float(b[q]),
+                                                  pl_f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+    return c + ((p[0] + p[1]) + (p[2] + p[3]));
+  } else {
+    return pl_mfma_chunk<DT>(a, b, c);
+  }
+}
+
 // ---------------------------------------------------------------- host side
 void pl_set_error(const char* fmt, ...);
 int pl_launch_status(const char* what);

@@ -5,11 +5,15 @@
 //
 // The 16 waves split K, so that for K up to 1024 a wave's whole K range (and
 // for K = 4096 half of it) is one round trip; their partials meet in LDS, summed
-// in wave order and rounded once to the model dtype; then every wave expands
+// pairwise and rounded once to the model dtype; then every wave expands
 // 128 bytes of each of the tile's y rows per step.  The first step's B and y
 // loads need nothing from the shrink and issue right behind its first loads, so
 // the expand waits on LDS only.  Products are MFMA with fp32 sums and the
-// epilogue is the expand's, as in the other fused kernel.
+// epilogue is the expand's, as in the other fused kernel.  In fp32 the sums over K
+// are kept in short chains, so that they are no less exact than a lane's share
+// of K and a tree over 64 lanes (delta against 64 bits, K = 2048, rank 16: 1.2e-7, a
+// wave per row 1.4e-7, one running sum per wave 2.3e-7; 64 x 60 rows, 2048 ->
+// 1024, rank 16: 24 us, a wave per row 155 us).
 //
 // Tiles are 16 consecutive positions of one batch row, straight from the
 // row -> slot map and the row lengths, with no plan and no scratch, at any K,
@@ -183,7 +187,7 @@ __global__ __launch_bounds__(kWThreads) void pl_lora_wide_rows(pl_wide_args a) {
 #pragma unroll
       for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
-        for (int cc = 0; cc < kWCC; ++cc) acc[jt] = pl_mfma_chunk<DT>(xf[cc], af[jt][cc], acc[jt]);
+        for (int cc = 0; cc < kWCC; ++cc) acc[jt] = pl_mfma_chunk_short<DT>(xf[cc], af[jt][cc], acc[jt]);
     };
     pl_u32x4 xf[kWCC], af[JT][kWCC];
     load_k(xf, af, k0);
@@ -210,11 +214,11 @@ __global__ __launch_bounds__(kWThreads) void pl_lora_wide_rows(pl_wide_args a) {
         const T* __restrict__ Aj = A + (j < rank ? pl_tile_off<DT>(j, kt, rank, K) : 0);
 #pragma unroll
         for (int q = 0; q < E; ++q) ae[q] = (j < rank && q < n) ? Aj[q] : (T)0.f;
-        acc[jt] = pl_mfma_chunk<DT>(__builtin_bit_cast(pl_u32x4, xe), __builtin_bit_cast(pl_u32x4, ae), acc[jt]);
+        acc[jt] = pl_mfma_chunk_short<DT>(__builtin_bit_cast(pl_u32x4, xe), __builtin_bit_cast(pl_u32x4, ae), acc[jt]);
       }
     }
 
-    // the 16 wave partials summed in wave order, rounded once to T;
+    // the 16 wave partials summed pairwise, rounded once to T;
     // acc[jt][v] holds (token 4*lg+v, rank rb + jt*16 + li)
     if (rb > 0) __syncthreads();  // the previous pass's sums are read
 #pragma unroll
@@ -224,11 +228,15 @@ __global__ __launch_bounds__(kWThreads) void pl_lora_wide_rows(pl_wide_args a) {
       const int jt = tid >> 8;
       const int l = (tid >> 2) & 63;
       const int v = tid & 3;
-      float sum = lds.red[0][jt][l][v];
+      float p[kWWaves];
 #pragma unroll
-      for (int w = 1; w < kWWaves; ++w) sum += lds.red[w][jt][l][v];
+      for (int w = 0; w < kWWaves; ++w) p[w] = lds.red[w][jt][l][v];
+#pragma unroll
+      for (int h = kWWaves / 2; h > 0; h /= 2)
+#pragma unroll
+        for (int w = 0; w < h; ++w) p[w] += p[w + h];
       const int j = rb + jt * 16 + (l & 15);
-      tt[((l >> 4) * 4 + v) * S::kTRow + j] = (T)(j < rank ? sum : 0.f);
+      tt[((l >> 4) * 4 + v) * S::kTRow + j] = (T)(j < rank ? p[0] : 0.f);
     } else if (kPass < kInstr && tid < JT * 256 + 16 * (kInstr - kPass)) {
       // the ranks past the pass that an expand block reads: zeros, until a later pass writes them
       const int i = tid - JT * 256;

@@ -73,3 +73,26 @@ def test_row_kernel_edges_match_the_oracle(gpu, dtype, rows, row_len, K, N, rank
         gaps = torch.ones(around.numel(), dtype=torch.bool)
         gaps[1:].as_strided(dy.shape, dy.stride()).fill_(False)
         assert torch.equal(around.view(-1).cpu()[gaps], torch.full((int(gaps.sum()),), 7.0, dtype=dtype))
+
+@pytest.mark.parametrize("K,rank", [(192, 4), (768, 16), (2000, 16), (4096, 64)])
+def test_row_kernel_fp32_sums_in_short_chains(gpu, K, rank):
+    """The delta's rms error against 64 bits stays below 0.42 * 2^-24 * sqrt(additions of one sum).
+
+    An addition rounds by 2^-24 / sqrt(3) of its power of two, 0.42 * 2^-24 of the running sum on average, independently
+    of the others.  The shrink adds 4 products, 4 words, K / 256 chunks and 16 waves pairwise (4 + 2 + K / 256 + 4), the
+    expand `rank` products.  One running sum over each wave's K / 16 elements and the waves in turn is past the
+    bound (1.06e-7, 1.62e-7, 2.25e-7 and 3.25e-7 for these sizes).
+    """
+    print("case:", K, rank, flush=True)
+    g = torch.Generator().manual_seed(K + rank)
+    N, tokens = 512, 256
+    layer = peft_layer(g, K, N, rank, 2.0 * rank)
+    cache = make_cache({"a": {"m": layer}}, {"m": (K, N)}, 1, rank, gpu, torch.float32, tiled=False)
+    slots = cache.ensure_resident(["a"])
+    x = torch.randn(tokens, K, generator=g)
+    y = torch.zeros(tokens, N, device=gpu)
+    seq = torch.tensor([tokens], dtype=torch.int32, device=gpu)
+    sgmv.lora_apply_rows(x.to(gpu), y, cache, "m", slots, seq, tokens)
+    want = 2.0 * ((x.double() @ layer[0].double().T) @ layer[1].double().T)
+    err = float((y.cpu().double() - want).norm() / want.norm())
+    assert err < 0.42 * 2.0**-24 * (10 + K / 256 + rank) ** 0.5, err
