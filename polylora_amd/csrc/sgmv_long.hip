@@ -8,13 +8,13 @@
 // read-modify-write wants (a probe over 705 MB of 28 KB rows: 5.7 TB/s with
 // 2 KB of each row per workgroup, 5.0 TB/s when a workgroup walks whole
 // rows).  Against one fused launch, whose workgroups run both phases, the
-// second launch costs about 5 us, and that is paid back once the outputs are
-// about 112 MB of traffic (the rule of sgmv.long_ok).  bf16, before -> after:
+// second launch costs about 5 us, and that is paid back from about 112 MB of
+// output traffic on, above rank 32 from 40 MB of x and y (sgmv.long_ok).  bf16, before -> after:
 //   4096 -> 2 x 14336, rank 32, 24740 tokens  642 -> 564 us (5.4 TB/s in the expand)
 //   2048 -> 8192, rank 64, 4593 tokens         78 -> 46 us
 //   14336 -> 4096, rank 32, 24740 tokens      268 -> 230 us
 // and against the split shrink and expand above rank 64:
-//   4096 -> 4096, rank 128, 4138 tokens        70 -> 48 us
+//   4096 -> 4096, rank 128, 4138 tokens        68 -> 43 us
 //   14336 -> 4096, rank 128, 11557 tokens     338 -> 182 us
 //
 // Both kernels work on units of consecutive 16-token tiles of one XCD's plan
@@ -28,6 +28,10 @@
 // of its operands.  Splitting K over workgroups (fp32 planes, summed by the
 // last to arrive) was slower at every size; 8 waves per workgroup left fewer,
 // larger workgroups to balance over the CUs (rank 32 prefill 578 against 564 us).
+//
+// In fp32 the sums over K are kept in short chains (K = 4096, error of the delta
+// against 64 bits: rank 64 2.1e-7, the fused launch 5.9e-7; rank 128 2.5e-7,
+// the split pair 3.5e-7; 6.0e-7 with one running sum per wave).
 #include <algorithm>
 
 #include "pl_common.h"
@@ -212,7 +216,7 @@ __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int jo
 #pragma unroll
       for (int jt = 0; jt < JT; ++jt)
 #pragma unroll
-        for (int cc = 0; cc < kCC; ++cc) acc[rt][jt] = pl_mfma_chunk<DT>(xm[cc], am[jt][cc], acc[rt][jt]);
+        for (int cc = 0; cc < kCC; ++cc) acc[rt][jt] = pl_mfma_chunk_short<DT>(xm[cc], am[jt][cc], acc[rt][jt]);
     }
   };
   // the waves take K steps in turn; a step past the range loads only zeros

@@ -100,3 +100,27 @@ def test_the_dispatch_takes_the_long_path_where_its_rule_says(gpu, monkeypatch):
             op(x.to(gpu).view(-1, 64), y)
             torch.testing.assert_close(y.cpu().view(base.shape), ref, **tol_for(torch.bfloat16))
         assert calls == want, (rank, rows, n)
+
+
+@pytest.mark.parametrize("K,rank", [(768, 8), (4096, 64), (4096, 128)])
+def test_long_fp32_sums_in_short_chains(gpu, K, rank):
+    """The delta's rms error against 64 bits stays below 0.42 * 2^-24 * sqrt(additions of one sum).
+
+    An addition rounds by 2^-24 / sqrt(3) of its power of two, 0.42 * 2^-24 of the running sum on average, independently
+    of the others.  The shrink adds 4 products, 4 words, K / 64 chunks and 4 waves (4 + 2 + K / 64 + 3), the expand
+    `rank` products.  One running sum over each wave's K / 4 elements is past the bound (2.6e-7, 5.9e-7 and 6.0e-7).
+    """
+    print("case:", K, rank, flush=True)
+    g = torch.Generator().manual_seed(K + rank)
+    N, tokens = 512, 1024
+    layer = peft_layer(g, K, N, rank, 2.0 * rank)
+    cache = make_cache({"a": {"m": layer}}, {"m": (K, N)}, 1, rank, gpu, torch.float32)
+    slots = cache.ensure_resident(["a"])
+    x = torch.randn(tokens, K, generator=g)
+    y = torch.zeros(tokens, N, device=gpu)
+    seq = torch.tensor([tokens], dtype=torch.int32, device=gpu)
+    plan = sgmv.SgmvPlan(slots, seq, tokens, cache.num_slots, distinct_slots=1)
+    sgmv.lora_long_stacked(x.to(gpu), [y], cache, ["m"], plan)
+    want = 2.0 * ((x.double() @ layer[0].double().T) @ layer[1].double().T)
+    err = float((y.cpu().double() - want).norm() / want.norm())
+    assert err < 0.42 * 2.0**-24 * (9 + K / 64 + rank) ** 0.5, err
