@@ -519,8 +519,10 @@ def fused_ok(plan: SgmvPlan, cache, in_features: int) -> bool:
 #   10.0 / 12.1), twice that for several modules, which share a tile's x
 #   (2048 -> 2048, 512, 512, 65 MB 25.4 / 25.7).
 # Above rank 64 the other choice is the split pair, slower from
-# LONG_MIN_TOKENS on (4096 -> 4096 rank 128, 1024 tokens 19.3 / 21.5 us, 2048
-# tokens 33.3 / 28.8).
+# LONG_MIN_TOKENS on in 16 bits (4096 -> 4096 rank 128, 1024 tokens 19.3 / 21.5
+# us, 2048 tokens 33.3 / 28.8), and the faster one in fp32 (rank 128, 4200 of 5600
+# tokens, 4096 -> 4096 114 / 135 us, 14336 -> 4096 280 / 334; rank 96, 1024 ->
+# 4096 58 / 69).
 LONG_MAX_RANK = 256  # half of it in fp32
 LONG_MIN_Y_BYTES = 112 << 20
 LONG_MIN_BYTES = 40 << 20
@@ -535,7 +537,7 @@ def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules:
         return False
     es = cache.dtype.itemsize
     if rank > FUSED_MAX_RANK:
-        return rank <= LONG_MAX_RANK * 2 // max(2, es) and tokens >= LONG_MIN_TOKENS
+        return es == 2 and rank <= LONG_MAX_RANK and tokens >= LONG_MIN_TOKENS
     if in_features > FUSED_MAX_K:
         return False
     if rank <= 32:

@@ -627,3 +627,14 @@ def test_long_path_rule(rank, tokens, fin, fout, modules, want):
     assert sgmv.long_ok(Obj(distinct_slots=1, tokens_cap=tokens), cache, fin, fout, modules) == want
     assert not sgmv.long_ok(Obj(distinct_slots=None, tokens_cap=tokens), cache, fin, fout, modules)
     assert not sgmv.long_ok(Obj(distinct_slots=tokens // 32, tokens_cap=tokens), cache, fin, fout, modules)
+
+
+@pytest.mark.parametrize("rank", [65, 96, 128, 256])
+def test_long_path_rule_leaves_fp32_above_rank_64_to_the_split_pair(rank):
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    plan = Obj(distinct_slots=1, tokens_cap=8192)
+    assert sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.float16), 4096, 4096)
+    assert not sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.float32), 4096, 4096)
