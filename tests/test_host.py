@@ -638,3 +638,15 @@ def test_long_path_rule_leaves_fp32_above_rank_64_to_the_split_pair(rank):
     plan = Obj(distinct_slots=1, tokens_cap=8192)
     assert sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.float16), 4096, 4096)
     assert not sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.float32), 4096, 4096)
+
+
+@pytest.mark.parametrize("ldt,want", [(32, 16), (64, 16), (72, 8), (128, 8)])
+def test_few_groups_take_more_k_splits_up_to_rank_64(ldt, want):
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    lib = Obj(pl_shrink_planes=lambda *a: a[2], pl_shrink_workspace_bytes=lambda *a: 0)
+    plan = Obj(group_cap=13, group_tokens=16)
+    # rows of a size that no other test asks for: the geometry is kept per shape
+    assert sgmv._shrink_geometry(lib, 2, 14336, torch.float16, plan, 7654321, ldt, None)[0] == want
