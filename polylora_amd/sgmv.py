@@ -253,7 +253,9 @@ def lora_apply(
     the fused kernel (lora_fused) or, with more data or ranks above its
     limit, to the two-launch path (long_ok); other plans of 16-token groups
     to the one-launch decode kernel (lora_decode_stacked) where it is not
-    slower; all unless k_splits asks for the split pair;
+    slower and cache.decode_handoff allows its wait (decode_waits_timed_out
+    says what happens if one runs out); all unless k_splits asks for the
+    split pair;
     x / y that do not meet the tiled path's alignment go to the row-based HIP
     kernels.
     """
@@ -871,9 +873,10 @@ def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -
     the GPU needs less) and is about even on the GPU, except above rank 64,
     whose shrink passes all arrive on one counter (37 rows, 14336 -> 4096, rank
     128: 13.8 -> 15.4 us), and for many rows of wide outputs (256 rows, 4096 ->
-    14336, rank 64: 18.6 -> 19.5 us).
+    14336, rank 64: 18.6 -> 19.5 us).  Never with the cache's decode_handoff
+    switch off.
     """
-    return (plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
+    return (cache.decode_handoff and plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
             and (plan.tokens_cap < 256 or out_features <= 2 * in_features))
 
 

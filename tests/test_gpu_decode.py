@@ -253,3 +253,23 @@ def test_lora_apply_in_one_launch_equals_the_split_pair(gpu, monkeypatch, dtype,
     sgmv.lora_apply(x, got[:, :N], cache, "m", plan)
     assert torch.equal(got, want) and bool(launches) == one
     assert not sgmv.decode_waits_timed_out(gpu)
+
+
+def test_lora_apply_keeps_to_separate_launches_with_the_hand_off_off(gpu, monkeypatch):
+    """cache.decode_handoff = False: lora_apply runs the split pair, with the one launch's result bit for bit."""
+    launches = []
+    launch = sgmv._decode_launch
+    monkeypatch.setattr(sgmv, "_decode_launch", lambda *a: (launches.append(1), launch(*a))[1])
+    g = torch.Generator().manual_seed(79)
+    cache = make_cache({"a": {"m": peft_layer(g, 520, 264, 16, 32.0)}}, {"m": (520, 264)}, 1, 16, gpu, torch.bfloat16)
+    plan = sgmv.SgmvPlan(cache.ensure_resident(["a"] * 21), torch.ones(21, dtype=torch.int32, device=gpu), 1,
+                         cache.num_slots, distinct_slots=1)
+    x = torch.randn(21, 520, generator=g).bfloat16().to(gpu)
+    base = torch.randn(21, 264, generator=g).bfloat16().to(gpu)
+    outs = []
+    for on in (False, True):
+        cache.decode_handoff = on
+        outs.append(sgmv.lora_apply(x, base.clone(), cache, "m", plan))
+        assert len(launches) == on
+    assert torch.equal(*outs) and not torch.equal(outs[0], base)
+    assert not sgmv.decode_waits_timed_out(gpu)

@@ -650,3 +650,14 @@ def test_few_groups_take_more_k_splits_up_to_rank_64(ldt, want):
     plan = Obj(group_cap=13, group_tokens=16)
     # rows of a size that no other test asks for: the geometry is kept per shape
     assert sgmv._shrink_geometry(lib, 2, 14336, torch.float16, plan, 7654321, ldt, None)[0] == want
+
+
+def test_lora_apply_takes_no_hand_off_where_the_cache_turns_it_off():
+    """cache.decode_handoff = False: lora_apply runs separate launches, as the wrapped Linears do."""
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    plan = Obj(group_tokens=16, tokens_cap=8)
+    assert sgmv._one_launch_ok(plan, Obj(rank8_cap=16, decode_handoff=True), 1024, 1024)
+    assert not sgmv._one_launch_ok(plan, Obj(rank8_cap=16, decode_handoff=False), 1024, 1024)
