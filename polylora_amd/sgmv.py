@@ -866,6 +866,9 @@ def lora_decode_stacked(x: torch.Tensor, ys: list, cache, module_names: list, pl
     return ys
 
 
+_ONE_LAUNCH_MAX_TOKENS = 8192
+
+
 def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -> bool:
     """Whether lora_apply runs one pl_lora_decode_stacked launch instead of the split pair.
 
@@ -873,10 +876,17 @@ def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -
     the GPU needs less) and is about even on the GPU, except above rank 64,
     whose shrink passes all arrive on one counter (37 rows, 14336 -> 4096, rank
     128: 13.8 -> 15.4 us), and for many rows of wide outputs (256 rows, 4096 ->
-    14336, rank 64: 18.6 -> 19.5 us).  Never with the cache's decode_handoff
-    switch off.
+    14336, rank 64: 18.6 -> 19.5 us).  Measured, and taken, up to the tokens
+    from which plans have 64-token groups (on the GPU, 150 adapters of rank
+    64: 4096 -> 4096, 2047 tokens 34.6 -> 33.4 us, 8191 tokens 84.0 -> 83.6;
+    14336 -> 4096, 4095 tokens 104 -> 97; 1024 -> 1024, 8191 tokens 28.1 ->
+    24.9; the worst of 110 sizes 512 tokens of 8 adapters, 14336 -> 4096, 21.8
+    -> 22.7): a 16-token plan of more tokens keeps the split pair, whose
+    workgroups wait for nothing.  Never with the cache's decode_handoff switch
+    off.
     """
     return (cache.decode_handoff and plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
+            and plan.tokens_cap < _ONE_LAUNCH_MAX_TOKENS
             and (plan.tokens_cap < 256 or out_features <= 2 * in_features))
 
 

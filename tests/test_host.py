@@ -661,3 +661,15 @@ def test_lora_apply_takes_no_hand_off_where_the_cache_turns_it_off():
     plan = Obj(group_tokens=16, tokens_cap=8)
     assert sgmv._one_launch_ok(plan, Obj(rank8_cap=16, decode_handoff=True), 1024, 1024)
     assert not sgmv._one_launch_ok(plan, Obj(rank8_cap=16, decode_handoff=False), 1024, 1024)
+
+
+def test_lora_apply_takes_one_launch_below_8192_tokens_only():
+    """16-token plans of more tokens (many adapters, or group_tokens=16 asked for) keep the split pair."""
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    cache = Obj(rank8_cap=64, decode_handoff=True)
+    assert sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=8191), cache, 4096, 4096)
+    assert not sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=8192), cache, 4096, 4096)
+    assert not sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=1 << 20), cache, 64, 64)
