@@ -134,6 +134,13 @@ const char* pl_last_error(void);
  * that the caller's allocator and this library share one HIP runtime. */
 int pl_is_device_pointer(const void* ptr);
 
+/* Id of the capture `stream` is recording into a HIP graph, another one for
+ * every capture; 0 when it records none, -1 when it records one of unknown
+ * id or the runtime cannot say.  For buffers that must hold values before a
+ * kernel runs: what a capture records happens at every replay of its graph
+ * and not before. */
+int64_t pl_stream_capture_id(void* stream);
+
 /* Group records a plan for `rows` rows of `row_len` tokens over `num_slots`
  * slots needs: at most n = ceil(rows*row_len/group_tokens) + num_slots - 1
  * groups, placed below 8 * ceil(n / 8). */

@@ -120,6 +120,7 @@ _SIGNATURES: dict[str, tuple] = {
         c_int32, c_void_p, c_void_p, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_int32, c_void_p,
     ),
     "pl_host_copy_async": (c_void_p, c_void_p, c_int64, c_void_p),
+    "pl_stream_capture_id": (c_void_p,),
     "pl_host_alloc": (c_int64,),
     "pl_host_free": (c_void_p,),
     "pl_slot_upload": (c_void_p, c_void_p, c_int64, c_void_p, c_void_p, c_int64, c_void_p),
@@ -127,7 +128,8 @@ _SIGNATURES: dict[str, tuple] = {
 }
 _RESTYPES = {"pl_last_error": ctypes.c_char_p, "pl_plan_group_capacity": c_int64, "pl_shrink_workspace_bytes": c_int64,
              "pl_host_alloc": c_void_p, "pl_sgmv_ref_workspace_bytes": c_int64, "pl_decode_counter_ints": c_int64,
-             "pl_sgmv_ref_part_bytes": c_int64, "pl_lora_long_workspace_bytes": c_int64}
+             "pl_sgmv_ref_part_bytes": c_int64, "pl_lora_long_workspace_bytes": c_int64,
+             "pl_stream_capture_id": c_int64}
 
 EXPORTED_SYMBOLS = tuple(_SIGNATURES)
 

@@ -43,6 +43,19 @@ extern "C" int pl_is_device_pointer(const void* ptr) {
   return (attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged) ? 1 : 0;
 }
 
+extern "C" int64_t pl_stream_capture_id(void* stream) {
+  hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+  unsigned long long id = 0;
+  const hipError_t err = hipStreamGetCaptureInfo(reinterpret_cast<hipStream_t>(stream), &status, &id);
+  if (err != hipSuccess) {
+    (void)hipGetLastError();
+    pl_set_error("hipStreamGetCaptureInfo: %s", hipGetErrorString(err));
+    return -1;
+  }
+  if (status == hipStreamCaptureStatusNone) return 0;
+  return (int64_t)id > 0 ? (int64_t)id : -1;
+}
+
 // Page-locked host memory of exactly `nbytes` (the caching host allocators
 // of frameworks round requests up, e.g. to powers of two, which matters when
 // adapter images fill most of the page-lockable memory).  A failed

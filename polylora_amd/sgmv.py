@@ -19,6 +19,7 @@ There is no CPU path: CPU tensors raise.
 from __future__ import annotations
 
 import ctypes
+from collections import deque
 
 import torch
 
@@ -769,25 +770,52 @@ class _HandoffCounters:
     allocated for the life of the process, so a HIP graph that recorded a
     launch keeps a valid pointer.  Word 0 is the status a timed-out wait sets
     to 1.
+
+    A clear made while a HIP graph is being captured runs only when that
+    graph is replayed.  A capture that needs counters the stream has not
+    cleared before therefore gets a buffer of its own, cleared inside the
+    graph and used by the launches of that capture alone (the last
+    CAPTURES_KEPT of them stay allocated for decode_waits_timed_out).
     """
+
+    CAPTURES_KEPT = 32
 
     def __init__(self, device: torch.device) -> None:
         self.device = device
         self.buf: torch.Tensor | None = None
         self.retired: list[torch.Tensor] = []
+        self.captured: deque = deque(maxlen=self.CAPTURES_KEPT)  # (capture id, buffer), newest last
 
     def get(self, ints: int) -> torch.Tensor:
-        if self.buf is None or self.buf.numel() < ints:
-            if self.buf is not None:
-                self.retired.append(self.buf)
-                ints = max(ints, 2 * self.buf.numel())
-            # cleared by a fill kernel on the current stream (the launch's stream),
-            # which a HIP graph being captured records like any other kernel; an
-            # ordinary tensor even under torch.inference_mode, so that
-            # decode_waits_timed_out can clear it outside that mode
-            with torch.inference_mode(False):
-                self.buf = torch.empty(max(64, ints), dtype=torch.int32, device=self.device).zero_()
+        if self.buf is not None and self.buf.numel() >= ints:
+            return self.buf
+        capture = _capture_id(self.device)
+        if capture:
+            if capture < 0 or not self.captured or self.captured[-1][0] != capture or self.captured[-1][1].numel() < ints:
+                self.captured.append((capture, self._cleared(ints)))
+            return self.captured[-1][1]
+        if self.buf is not None:
+            self.retired.append(self.buf)
+            ints = max(ints, 2 * self.buf.numel())
+        self.buf = self._cleared(ints)
         return self.buf
+
+    def _cleared(self, ints: int) -> torch.Tensor:
+        # cleared by a fill kernel on the current stream (the launch's stream),
+        # which a HIP graph being captured records like any other kernel; an
+        # ordinary tensor even under torch.inference_mode, so that
+        # decode_waits_timed_out can clear it outside that mode
+        with torch.inference_mode(False):
+            return torch.empty(max(64, ints), dtype=torch.int32, device=self.device).zero_()
+
+    def buffers(self) -> list:
+        """The buffers that launches may be using, for decode_waits_timed_out."""
+        return ([] if self.buf is None else [self.buf]) + [buf for _, buf in self.captured]
+
+
+def _capture_id(device: torch.device) -> int:
+    """pl_stream_capture_id of the device's current stream."""
+    return int(_native.load().pl_stream_capture_id(_stream(device)))
 
 
 _COUNTERS: dict[tuple[int, int], _HandoffCounters] = {}
@@ -816,13 +844,15 @@ def decode_waits_timed_out(device: torch.device | None = None, clear: bool = Tru
     launch's shrink takes."""
     hit = False
     for (index, _), c in _COUNTERS.items():
-        if c.buf is None or (device is not None and c.device != torch.device(device)):
+        bufs = c.buffers()
+        if not bufs or (device is not None and c.device != torch.device(device)):
             continue
         torch.cuda.synchronize(c.device)
-        if int(c.buf[0]) != 0:
-            hit = True
-            if clear:
-                c.buf.zero_()  # no launch is in flight on the device: every counter can be reset
+        for buf in bufs:
+            if int(buf[0]) == 1:  # a captured buffer holds anything until its graph has run
+                hit = True
+                if clear:
+                    buf.zero_()  # no launch is in flight on the device: every counter can be reset
     return hit
 
 

@@ -273,3 +273,54 @@ def test_lora_apply_keeps_to_separate_launches_with_the_hand_off_off(gpu, monkey
         assert len(launches) == on
     assert torch.equal(*outs) and not torch.equal(outs[0], base)
     assert not sgmv.decode_waits_timed_out(gpu)
+
+
+def test_graphs_captured_on_one_stream_replay_in_any_order(gpu, monkeypatch):
+    """Two graphs of lora_apply and lora_decode_stacked captured one after the other on a stream without counters yet:
+    the second replayed first, then both in turn with eager launches between them, equal to the eager results."""
+    _announce(test="two_graphs")
+    monkeypatch.setattr(sgmv, "_COUNTERS", {})  # no stream has counters: both captures need cleared ones
+    g = torch.Generator().manual_seed(80)
+    shapes = {"q": (1024, 512), "k": (1024, 264)}
+    adapters = {f"a{i}": {m: peft_layer(g, fi, fo, r, 2.0 * r) for m, (fi, fo) in shapes.items()}
+                for i, r in enumerate([8, 64])}
+    cache = make_cache(adapters, shapes, 2, 64, gpu, torch.bfloat16)
+    runs = []
+    for rows in (20, 45):
+        slots = cache.ensure_resident([["a0", "a1", "__base__"][i] for i in torch.randint(0, 3, (rows,), generator=g).tolist()])
+        plan = sgmv.SgmvPlan(slots, torch.ones(rows, dtype=torch.int32, device=gpu), 1, cache.num_slots, distinct_slots=2)
+        x = torch.randn(rows, 1024, generator=g).bfloat16().to(gpu)
+        base = [torch.randn(rows, n, generator=g).bfloat16().to(gpu) for n in (512, 264)]
+        runs.append((plan, x, base, [torch.empty_like(b) for b in base]))
+
+    def step(run, ys):
+        plan, x, base, _ = run
+        for y, b in zip(ys, base):
+            y.copy_(b)
+        sgmv.lora_apply(x, ys[0], cache, "q", plan)
+        sgmv.lora_decode_stacked(x, ys, cache, ["q", "k"], plan)
+
+    torch.cuda.synchronize()
+    graphs = []
+    for run in runs:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            step(run, run[3])
+        graphs.append(graph)
+    want = [[torch.empty_like(b) for b in run[2]] for run in runs]
+    for run, ys in zip(runs, want):
+        step(run, ys)
+    torch.cuda.synchronize()
+    for i in (1, 0, 1, 1, 0):
+        for y in runs[i][3]:
+            y.fill_(-1.0)
+        graphs[i].replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(runs[i][3], want[i])), i
+        again = [torch.empty_like(b) for b in runs[i][2]]
+        step(runs[i], again)  # eager work between the replays
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(again, want[i])), i
+    assert not sgmv.decode_waits_timed_out(gpu)
+    captures = [capture for c in sgmv._COUNTERS.values() for capture, _ in c.captured]
+    assert len(captures) == 4 and len(set(captures)) == 2  # in each: for one module, then for two

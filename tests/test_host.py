@@ -673,3 +673,33 @@ def test_lora_apply_takes_one_launch_below_8192_tokens_only():
     assert sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=8191), cache, 4096, 4096)
     assert not sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=8192), cache, 4096, 4096)
     assert not sgmv._one_launch_ok(Obj(group_tokens=16, tokens_cap=1 << 20), cache, 64, 64)
+
+
+def test_counters_cleared_inside_a_capture_serve_that_capture_alone(monkeypatch):
+    """A clear recorded into a HIP graph has not run when the capture ends: neither another capture on the stream nor
+    an eager call may take that buffer for cleared."""
+    from polylora_amd import sgmv
+
+    capture = [7]
+    monkeypatch.setattr(sgmv, "_capture_id", lambda device: capture[0], raising=False)
+    c = sgmv._HandoffCounters(torch.device("cpu"))
+    first = c.get(64)
+    assert c.get(64) is first  # launches of one capture share its counters
+    more = c.get(4096)
+    assert more is not first and more.numel() >= 4096
+    capture[0] = 8
+    second = c.get(64)
+    assert second is not first and second is not more
+    capture[0] = 0
+    eager = c.get(64)
+    assert all(eager is not b for b in (first, more, second)) and not bool(eager.any())
+    capture[0] = 9
+    assert c.get(64) is eager  # cleared before the capture: its launches leave it at zero
+    grown = c.get(1 << 16)
+    capture[0] = 0
+    assert grown is not eager and c.get(64) is eager and c.get(1 << 16) is not grown
+    capture[0] = -1  # a capture of unknown id shares nothing
+    assert c.get(1 << 20) is not c.get(1 << 20)
+    for capture[0] in range(100, 200):
+        c.get(1 << 20)
+    assert len(c.captured) == c.CAPTURES_KEPT
