@@ -716,27 +716,6 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   }
   const int sub = group_tokens / 16;
   const int64_t tiles = (group_cap + kXcds - 1) / kXcds * kXcds * sub;
-  if (n_chunks > 1 << 24 || !pl_grid_fits(tiles * n_modules, 64 * kLWaves) ||
-      !pl_grid_fits(tiles * n_chunks, 64 * kLWaves) || tiles * n_chunks > 0x7fffffff) {
-    pl_set_error("pl_lora_long: grid of %lld groups too large", (long long)group_cap);
-    return PL_ERR_LIMIT;
-  }
-  if (group_cap == 0) return PL_OK;
-  a.x = x;
-  a.ldx = ldx;
-  a.K = K;
-  a.arena = reinterpret_cast<const char*>(arena);
-  a.table = table;
-  a.num_modules = num_modules;
-  a.tok = tok;
-  a.groups = groups;
-  a.meta = meta;
-  a.group_cap = (int32_t)group_cap;
-  a.sub = sub;
-  a.epilogue = epilogue;
-  a.n_jobs = n_modules;
-  a.n_chunks = (int32_t)n_chunks;
-  a.ldt = long_ldt(ldt);
   // Shrink: two tiles per workgroup share each A load once the launch has
   // 512 tiles (8192 tokens), above rank 64 from 320 on; below, one tile, for
   // more workgroups (bf16, K = 4096: rank 32 with 260 tiles 12 against 17 us, 520
@@ -759,6 +738,27 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   for (int j = 0; j < n_modules; ++j) lines = lines && (ldy[j] * es) % 128 == 0;
   const int unit = !lines || tiles * n_chunks < 2048 ? 1 : ldt > 32 ? 4 : 2;
   a.passes = (ldt + 16 * jt - 1) / (16 * jt);
+  a.sub = sub;
+  a.group_cap = (int32_t)group_cap;
+  a.n_jobs = n_modules;
+  a.n_chunks = (int32_t)n_chunks;
+  if (n_chunks > 1 << 24 || !pl_grid_fits(long_units(a, rt) * kXcds * n_modules * a.passes, 64 * kLWaves) ||
+      !pl_grid_fits(long_units(a, unit) * kXcds * n_chunks, 64 * kLWaves)) {
+    pl_set_error("pl_lora_long: grid of %lld groups too large", (long long)group_cap);
+    return PL_ERR_LIMIT;
+  }
+  if (group_cap == 0) return PL_OK;
+  a.x = x;
+  a.ldx = ldx;
+  a.K = K;
+  a.arena = reinterpret_cast<const char*>(arena);
+  a.table = table;
+  a.num_modules = num_modules;
+  a.tok = tok;
+  a.groups = groups;
+  a.meta = meta;
+  a.epilogue = epilogue;
+  a.ldt = long_ldt(ldt);
   hipStream_t s = reinterpret_cast<hipStream_t>(stream);
   switch (dtype) {
     case PL_BF16:

@@ -547,12 +547,19 @@ def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules:
     es = cache.dtype.itemsize
     if rank > FUSED_MAX_RANK:
         return es == 2 and rank <= LONG_MAX_RANK and tokens >= LONG_MIN_TOKENS
-    if in_features > FUSED_MAX_K:
+    if in_features > FUSED_MAX_K or not _long_grid_fits(tokens, es, rank, out_features, modules):
         return False
     if rank <= 32:
         return 2 * es * tokens * out_features >= LONG_MIN_Y_BYTES
     return (es * (in_features + out_features) >= LONG_MIN_ROW_BYTES
             and es * tokens * (in_features + 2 * out_features) >= LONG_MIN_BYTES * min(modules, 2))
+
+
+def _long_grid_fits(tokens: int, es: int, rank: int, out_features: int, modules: int) -> bool:
+    """Whether pl_lora_long_stacked can launch what the fused kernel can: its expand has a workgroup for every tile and
+    1024 bytes of a y row (512 above two rank steps), the fused kernel one for every tile and module."""
+    chunks = es * out_features // (1024 if rank * es <= 128 else 512) + modules
+    return (tokens // 16 + 4 * _native.PL_MAX_SLOTS + 64) * chunks < 1 << 24
 
 
 def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, out_features: int, stream: int | None, modules: int = 1) -> bool:

@@ -703,3 +703,36 @@ def test_counters_cleared_inside_a_capture_serve_that_capture_alone(monkeypatch)
     for capture[0] in range(100, 200):
         c.get(1 << 20)
     assert len(c.captured) == c.CAPTURES_KEPT
+
+
+def test_long_path_counts_its_rank_passes_in_the_size_check():
+    """pl_lora_long_stacked refuses a launch whose workgroups do not fit, rank passes included, before any HIP call."""
+    lib = _native.load()
+    fake = [ctypes.c_void_p(4096 * (i + 1)) for i in range(6)]  # 16-byte aligned, never dereferenced
+
+    def call(group_cap, ldt):
+        tokens = 16 * group_cap
+        one = lambda t, v: (t * 1)(v)  # noqa: E731
+        return lib.pl_lora_long_stacked(
+            _native.PL_BF16, fake[0], 8, 8, 1, one(ctypes.c_int32, 0), one(ctypes.c_void_p, 4096 * 9),
+            one(ctypes.c_int64, 8), one(ctypes.c_int32, 8), fake[1], fake[2], 1, ldt, fake[3], fake[4], fake[5],
+            group_cap, 16, tokens, one(ctypes.c_void_p, 4096 * 10), lib.pl_lora_long_workspace_bytes(_native.PL_BF16, tokens, ldt),
+            _native.PL_EPI_FALLBACK, None)
+
+    # 10M tiles of one column chunk: the expand fits, and so do 5M shrink workgroups, but not four passes of them
+    assert call(10_000_000, 256) == _native.PL_ERR_LIMIT and b"too large" in lib.pl_last_error()
+    assert call((1 << 24) + 1, 16) == _native.PL_ERR_LIMIT
+    assert call(0, 256) == _native.PL_OK  # nothing to do
+
+
+@pytest.mark.parametrize("tokens,fout,modules,rank,want", [
+    (1 << 20, 520, 1, 16, True), (1 << 27, 520, 1, 16, False), (1 << 27, 8, 1, 16, True), (1 << 27, 16, 2, 16, False),
+    (1 << 23, 16384, 1, 16, False), (1 << 24, 4096, 1, 64, True), (1 << 26, 4096, 1, 64, False)])
+def test_long_path_rule_stays_within_what_one_launch_can_hold(tokens, fout, modules, rank, want):
+    """Calls the fused kernel takes and the long path's grid cannot hold stay with the fused kernel."""
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    plan = Obj(distinct_slots=1, tokens_cap=tokens)
+    assert sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.bfloat16), 4096, fout, modules) == want
