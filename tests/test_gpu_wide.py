@@ -74,6 +74,7 @@ def test_row_kernel_edges_match_the_oracle(gpu, dtype, rows, row_len, K, N, rank
         gaps[1:].as_strided(dy.shape, dy.stride()).fill_(False)
         assert torch.equal(around.view(-1).cpu()[gaps], torch.full((int(gaps.sum()),), 7.0, dtype=dtype))
 
+
 @pytest.mark.parametrize("K,rank", [(192, 4), (768, 16), (2000, 16), (4096, 64)])
 def test_row_kernel_fp32_sums_in_short_chains(gpu, K, rank):
     """The delta's rms error against 64 bits stays below 0.42 * 2^-24 * sqrt(additions of one sum).
@@ -96,3 +97,33 @@ def test_row_kernel_fp32_sums_in_short_chains(gpu, K, rank):
     want = 2.0 * ((x.double() @ layer[0].double().T) @ layer[1].double().T)
     err = float((y.cpu().double() - want).norm() / want.norm())
     assert err < 0.42 * 2.0**-24 * (10 + K / 256 + rank) ** 0.5, err
+
+
+def _overlapping(kind, T, K, N, dtype, g, device):
+    """x [T, K] and y [T, N] in one buffer: y is x, beside it in packed rows, its last columns, or one row further."""
+    ld = {"same": K, "beside": K + N, "tail": K + 7, "next row": K}[kind]
+    buf = torch.randn(T + 1, ld, generator=g).to(dtype).to(device)
+    x = buf[:T, :K]
+    y = {"same": buf[:T, :N], "beside": buf[:T, K:], "tail": buf[:T, ld - N:], "next row": buf[1:, :N]}[kind]
+    return x, y
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("kind", ["same", "beside", "tail", "next row"])
+@pytest.mark.parametrize("rows,row_len,rank", [(3, 20, 16), (2, 7, 40)])
+def test_row_kernel_reads_x_before_an_overlapping_y(gpu, dtype, kind, rows, row_len, rank):
+    """y over x in one buffer gives what separate buffers give; wide outputs, so that a tile has several column ranges."""
+    print("case:", dtype, kind, rows, row_len, rank, flush=True)
+    g = torch.Generator().manual_seed(rank)
+    K, N, T = 2050, 2050, rows * row_len
+    cache = make_cache({"a": {"m": peft_layer(g, K, N, rank, 2.0 * rank)}}, {"m": (K, N)}, 1, rank, gpu, dtype, tiled=False)
+    slots = cache.ensure_resident(["a"] * rows)
+    seq = torch.full((rows,), row_len, dtype=torch.int32, device=gpu)
+    x, y = _overlapping(kind, T, K, N, dtype, g, gpu)
+    want = y.clone()
+    sgmv.lora_apply_rows(x.clone(), want, cache, "m", slots, seq, row_len)
+    sgmv.lora_apply_rows(x, y, cache, "m", slots, seq, row_len)
+    if kind == "next row":  # the plain kernels, whose sums have another order
+        torch.testing.assert_close(y, want, **tol_for(dtype))
+    else:
+        assert torch.equal(y, want)
