@@ -47,6 +47,7 @@ struct pl_long_args {
   const void* x;
   int64_t ldx;
   int32_t K;
+  int32_t kw;        // shrink: K per wave, whole pairs of steps; 0: steps in turn
   const char* arena;
   const pl_slot_entry* table;
   int32_t num_modules;
@@ -219,24 +220,28 @@ __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int jo
         for (int cc = 0; cc < kCC; ++cc) acc[rt][jt] = pl_mfma_chunk_short<DT>(xm[cc], am[jt][cc], acc[rt][jt]);
     }
   };
-  // the waves take K steps in turn; a step past the range loads only zeros
+  // the waves take shares of K (a.kw) or K steps in turn; a step past the
+  // range loads only zeros
   pl_u32x4 xa[2 * RT], aa[JT][kCC], xb[2 * RT], ab[JT][kCC];
-  constexpr int kTurn = kLWaves * kStep;
-  int kb = wave * kStep;
+  const int next = a.kw > 0 ? kStep : kLWaves * kStep;
+  const int k1 = a.kw > 0 ? min(K, (wave + 1) * a.kw) : K;
+  int kb = wave * (a.kw > 0 ? a.kw : kStep);
   load(xa, aa, kb);
-  for (; kb + 2 * kTurn < K; kb += 2 * kTurn) {
-    load(xb, ab, kb + kTurn);
+  for (; kb + 2 * next < k1; kb += 2 * next) {
+    load(xb, ab, kb + next);
     __builtin_amdgcn_sched_barrier(0);
     mfma(xa, aa);
-    load(xa, aa, kb + 2 * kTurn);
+    load(xa, aa, kb + 2 * next);
     __builtin_amdgcn_sched_barrier(0);
     mfma(xb, ab);
   }
-  load(xb, ab, kb + kTurn);
-  __builtin_amdgcn_sched_barrier(0);
-  mfma(xa, aa);
-  __builtin_amdgcn_sched_barrier(0);
-  mfma(xb, ab);
+  if (kb < k1) {
+    load(xb, ab, kb + next);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma(xa, aa);
+    __builtin_amdgcn_sched_barrier(0);
+    mfma(xb, ab);
+  }
 
   // the wave partials summed in wave order; acc[rt][jt][v] holds
   // (token 4*lg+v, rank rb + jt*16 + li)
@@ -751,6 +756,15 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   a.x = x;
   a.ldx = ldx;
   a.K = K;
+  // In 16 bits the ranks of the fused kernel get its shares of K per wave, so
+  // that each sum is the same additions in the same order and either kernel
+  // gives the same bits: a Linear alone and with its siblings may take
+  // different ones.  (Steps in turn instead: 32768 tokens, 4096 -> 14336, rank
+  // 32 280.6 us, shares 279.5; 4096 tokens, 14336 -> 4096, rank 64 52.0 and 53.1;
+  // above rank 64 turns, 8192 tokens, 8192 -> 2048, rank 256 85.7 and 87.3.)
+  const int64_t pair = 16 * E;
+  const int64_t share = ((int64_t)K + kLWaves - 1) / kLWaves;
+  a.kw = dtype != PL_F32 && ldt <= 64 ? (int32_t)((share + pair - 1) / pair * pair) : 0;
   a.arena = reinterpret_cast<const char*>(arena);
   a.table = table;
   a.num_modules = num_modules;

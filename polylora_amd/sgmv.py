@@ -562,9 +562,19 @@ def _long_grid_fits(tokens: int, es: int, rank: int, out_features: int, modules:
     return (tokens // 16 + 4 * _native.PL_MAX_SLOTS + 64) * chunks < 1 << 24
 
 
-def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, out_features: int, stream: int | None, modules: int = 1) -> bool:
-    """long_ok, on the current stream only: the workspace is allocated there."""
-    return long_ok(plan, cache, x.shape[1], out_features, modules) and stream in (None, _stream(x.device))
+def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, widths, stream: int | None) -> list:
+    """long_ok of each of the modules of output `widths` that share x, on the current stream only: the workspace is
+    allocated there.
+
+    A Linear gives the same bits alone and with its siblings: in 16 bits the
+    two paths do, so modules that share x decide together; in fp32, where the
+    long path's sums are the more exact, each decides as it does alone.
+    """
+    if stream not in (None, _stream(x.device)):
+        return [False] * len(widths)
+    if x.element_size() == 2:
+        return [long_ok(plan, cache, x.shape[1], sum(widths), len(widths))] * len(widths)
+    return [long_ok(plan, cache, x.shape[1], n) for n in widths]
 
 
 def _long_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, epilogue: int, stream: int) -> None:
@@ -650,7 +660,7 @@ def _fused_launch(x, y, cache, module_name: str, plan: SgmvPlan, epilogue: int, 
     """pl_lora_fused on operands the caller has checked, or the two-launch path where long_ok prefers it."""
     K, N = x.shape[1], y.shape[1]
     if slices is None:
-        if _use_long(x, plan, cache, N, stream):
+        if _use_long(x, plan, cache, (N,), stream)[0]:
             _long_launch(x, [y], cache, [module_name], plan, epilogue, stream)
             return
         slices = choose_slices(plan, N)
@@ -675,15 +685,23 @@ def lora_fused_stacked(
     """lora_fused for sibling Linears fed the same x, in one launch (pl_lora_fused_stacked): ys[i] in place.
 
     A tile's modules run side by side on one XCD, so x comes from HBM once.
-    As lora_fused, in two launches where long_ok prefers them.
+    As lora_fused, in two launches where long_ok prefers them (fp32: for the
+    modules for which it does).
     """
     _check_stacked(x, ys, cache, module_names, plan)
     if cache.rank8_cap > FUSED_MAX_RANK:
         raise ValueError(f"lora_fused takes ranks up to {FUSED_MAX_RANK}; the cache holds up to {cache.rank8_cap}")
-    if slices is None and _use_long(x, plan, cache, sum(y.shape[1] for y in ys), stream, len(ys)):
-        _long_launch(x, ys, cache, module_names, plan, epilogue, _stream(x.device))
-        return ys
     _, mods, widths, _ = _module_set(cache, module_names)
+    long = _use_long(x, plan, cache, widths, stream) if slices is None else [False]
+    if any(long):
+        picked = [i for i, ok in enumerate(long) if ok]
+        _long_launch(x, [ys[i] for i in picked], cache, [module_names[i] for i in picked], plan, epilogue,
+                     _stream(x.device))
+        rest = [i for i, ok in enumerate(long) if not ok]
+        if rest:
+            lora_fused_stacked(x, [ys[i] for i in rest], cache, [module_names[i] for i in rest], plan,
+                               epilogue=epilogue, stream=stream)
+        return ys
     arena, table, n_mod, _, ldt = _cache_args(cache, module_names[0])
     rc = _native.calls().pl_lora_fused_stacked(
         _native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), x.shape[1], len(ys), mods,

@@ -124,3 +124,64 @@ def test_long_fp32_sums_in_short_chains(gpu, K, rank):
     want = 2.0 * ((x.double() @ layer[0].double().T) @ layer[1].double().T)
     err = float((y.cpu().double() - want).norm() / want.norm())
     assert err < 0.42 * 2.0**-24 * (9 + K / 64 + rank) ** 0.5, err
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("rows,row_len,K,N,ranks", [
+    (4, 40, 8, 24, [1, 16]), (3, 70, 64, 520, [8, 15]), (5, 33, 136, 264, [17, 32, 3]), (2, 100, 520, 1032, [33, 64]),
+    (3, 50, 2056, 72, [16, 64, 40]), (2, 90, 4104, 512, [32, 5]), (40, 256, 1000, 136, [64, 16, 31])])
+def test_long_and_fused_paths_give_the_same_bits(gpu, dtype, rows, row_len, K, N, ranks):
+    """In 16 bits the two paths make every sum of the same additions in the same order, so a Linear's output does not
+    depend on which of them its call took: K around shares of one to several step pairs, ranks around a tile."""
+    print("case:", dtype, rows, row_len, K, N, ranks, flush=True)
+    g = torch.Generator().manual_seed(K + N)
+    adapters = {f"a{i}": {"m": peft_layer(g, K, N, r, 2.0 * r)} for i, r in enumerate(ranks)}
+    cache = make_cache(adapters, {"m": (K, N)}, len(ranks), max(ranks), gpu, dtype)
+    ids = list(adapters) + ["__base__"]
+    row_slot = cache.ensure_resident([ids[i] for i in torch.randint(0, len(ids), (rows,), generator=g).tolist()])
+    seq = torch.randint(0, row_len + 1, (rows,), generator=g, dtype=torch.int32).to(gpu)
+    x = torch.randn(rows * row_len, K, generator=g).to(dtype).to(gpu)
+    base = torch.randn(rows * row_len, N, generator=g).to(dtype).to(gpu)
+    for group_tokens in (16, 64):
+        plan = sgmv.SgmvPlan(row_slot, seq, row_len, cache.num_slots, distinct_slots=len(ranks), group_tokens=group_tokens)
+        fused = sgmv.lora_fused(x, base.clone(), cache, "m", plan, slices=1)
+        (long,) = sgmv.lora_long_stacked(x, [base.clone()], cache, ["m"], plan)
+        assert torch.equal(fused, long) and not torch.equal(fused, base)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("rank", [16, 64])
+def test_a_linear_alone_and_with_its_siblings_gives_the_same_bits(gpu, monkeypatch, dtype, rank):
+    """Sizes for which a Linear alone takes the fused kernel and with its siblings the long path (the first forward
+    runs Linears alone, later ones the learned siblings together): equal outputs, and both kernels really ran."""
+    ran = []
+    calls = sgmv._native.calls()
+
+    class Spy:
+        def __getattr__(self, name):
+            f = getattr(calls, name)
+            return lambda *a: (ran.append(name), f(*a))[1]
+
+    spy = Spy()
+    monkeypatch.setattr(sgmv._native, "calls", lambda: spy)
+    g = torch.Generator().manual_seed(rank)
+    K, shapes, tokens = 1000, {"q": 1536, "k": 264, "v": 264}, 1200
+    es = torch.empty((), dtype=dtype).element_size()
+    # thresholds between k or v alone and q alone or all together
+    monkeypatch.setattr(sgmv, "LONG_MIN_Y_BYTES", 2 * es * tokens * 1000)
+    monkeypatch.setattr(sgmv, "LONG_MIN_BYTES", es * tokens * 2500)
+    monkeypatch.setattr(sgmv, "LONG_MIN_ROW_BYTES", 0)
+    adapters = {f"a{i}": {m: peft_layer(g, K, n, r, 2.0 * r) for m, n in shapes.items()} for i, r in enumerate([rank, 5])}
+    cache = make_cache(adapters, {m: (K, n) for m, n in shapes.items()}, 2, rank, gpu, dtype)
+    slots = cache.ensure_resident(["a0", "a1", "a0"])
+    plan = sgmv.SgmvPlan(slots, torch.tensor([400, 333, 17], dtype=torch.int32, device=gpu), 400, cache.num_slots,
+                         distinct_slots=2)
+    x = torch.randn(tokens, K, generator=g).to(dtype).to(gpu)
+    bases = [torch.randn(tokens, n, generator=g).to(dtype).to(gpu) for n in shapes.values()]
+    alone = [sgmv.lora_apply(x, b.clone(), cache, m, plan) for m, b in zip(shapes, bases)]
+    assert ran == ["pl_lora_long_stacked", "pl_lora_fused", "pl_lora_fused"]
+    ran.clear()
+    together = sgmv.lora_fused_stacked(x, [b.clone() for b in bases], cache, list(shapes), plan)
+    assert ran[0] == "pl_lora_long_stacked" and len(ran) == (2 if dtype == torch.float32 else 1)
+    for m, a, b in zip(shapes, alone, together):
+        assert torch.equal(a, b), m
