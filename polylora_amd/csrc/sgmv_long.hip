@@ -726,11 +726,12 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   // more workgroups (bf16, K = 4096: rank 32 with 260 tiles 12 against 17 us, 520
   // tiles 16 against 13; rank 64 with 354 tiles 17.4 against 17.0, fewer of them
   // in use 13 against 18; rank 128 with 260 tiles 21 against 23, 354 tiles 24
-  // against 22).  Passes of 32 ranks balance better over the CUs than passes
+  // against 22; fp32 to rank 32 from 1024 on: 9152 -> 3072, rank 32, 512 tiles 128
+  // against 112, 896 tiles 186 against 173, 1024 tiles 195 against 213).  Passes of 32 ranks balance better over the CUs than passes
   // of 64 (rank 64, 520 tiles 16 against 18 us; K = 14336 44 against 56) until
   // they make 1536 workgroups, when rereading x costs more (K = 14336, rank 128,
   // 1040 tiles: 195 against 130 us).
-  const int rt = tiles >= (ldt > 64 ? 320 : 512) ? 2 : 1;
+  const int rt = tiles >= (ldt > 64 ? 320 : dtype == PL_F32 && ldt <= 32 ? 1024 : 512) ? 2 : 1;
   const int64_t blocks = tiles / rt * n_modules * ((ldt + 31) / 32);
   const int jt = ldt <= 16 ? 1 : ldt <= 32 || blocks < 1536 ? 2 : 4;
   // Expand: tiles per workgroup, which share the workgroup's B: 4 above rank

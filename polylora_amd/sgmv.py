@@ -513,30 +513,53 @@ def fused_ok(plan: SgmvPlan, cache, in_features: int) -> bool:
     return plan.tokens_cap >= 64 * max(1, distinct) and plan.tokens_cap >= 1024
 
 
-# Where pl_lora_long_stacked takes over from the fused launch.  Its second
-# launch costs about 5 us, which its faster streaming pays back
-# * up to rank 32, from LONG_MIN_Y_BYTES of y read and written on (y traffic of
-#   the plan's capacity, fused against long on MI355X, bf16 unless said: 2048 ->
-#   8192 rank 16, 67 MB 16.4 / 19.3 us, 134 MB 32.5 / 28.2; 4096 -> 4096 rank 32,
-#   67 MB 21.0 / 23.3, 134 MB 40.9 / 35.5; 4096 -> 2 x 14336 rank 16, 117 MB 28.4 /
-#   26.3; fp32 768 -> 3072 rank 8, 100 MB 20.6 / 22.5, 201 MB 37.4 / 35.4);
-# * above, where the fused launch rereads 64 ranks of A and B for every 16
+# Where pl_lora_long_stacked takes over from the fused launch.  Figures are us of
+# fused / long on the GPU, bf16 unless said, 83% of the tokens in use; the lines
+# were drawn over 4,091 sizes (768 to 14336 inputs, 128 to 14336 outputs, ranks
+# 8 to 64, one to three modules), at 92% of which the path they take is within
+# 5% of the faster one (with bytes alone as the rule at 86%, and up to 42% off
+# where it took the long path).
+#
+# Up to FUSED_ROUND_TOKENS the fused kernel's tiles all run in its first round,
+# one to a CU, and the long path's shrink has as few workgroups as tiles.  The
+# long path then pays only where the output is wide against the input, so that
+# the expand, which it splits over more workgroups, is most of the work.
+#
+# * Up to rank 32 its second launch costs about 5 us, which its faster streaming
+#   pays back from LONG_MIN_Y_BYTES of y read and written on (4096 -> 4096 rank 32,
+#   7168 tokens 41.4 / 39.8, 10240 tokens 59.2 / 53.5), below 4096 tokens of
+#   one module only for wide outputs (14336 -> 14336 rank 16, 2048 tokens 35.5 /
+#   47.2; 2048 -> 14336 rank 32, 3072 tokens 48.0 / 39.1).  At ranks to 16 and
+#   widths that fill the fused kernel's waves but not several workgroups of
+#   them, it takes twice the bytes, four times with a short K as well (2048 ->
+#   2048 rank 8, 14336 tokens 28.3 / 33.1, 28672 tokens 54.4 / 54.6; 768 -> 3 x 768
+#   rank 8, 126 MB 17% slower); in fp32 the like, at higher bytes.
+# * Above, where the fused launch rereads 64 ranks of A and B for every 16
 #   tokens, from LONG_MIN_BYTES of x and y on with rows of at least
-#   LONG_MIN_ROW_BYTES in all (rank 64: 4096 -> 4096, 2048 tokens 18.8 / 17.6 us,
-#   5600 tokens 29.3 / 26.5; 2048 -> 8192, 1024 tokens 16.2 / 17.3, 2560 tokens
-#   36.4 / 19.5; 14336 -> 4096, 2560 tokens 53.0 / 34.1; 1024 -> 1024, 5600 tokens
-#   10.0 / 12.1), twice that for several modules, which share a tile's x
-#   (2048 -> 2048, 512, 512, 65 MB 25.4 / 25.7).
-# Above rank 64 the other choice is the split pair, slower from
-# LONG_MIN_TOKENS on in 16 bits (4096 -> 4096 rank 128, 1024 tokens 19.3 / 21.5
-# us, 2048 tokens 33.3 / 28.8), and the faster one in fp32 (rank 128, 4200 of 5600
-# tokens, 4096 -> 4096 114 / 135 us, 14336 -> 4096 280 / 334; rank 96, 1024 ->
-# 4096 58 / 69).
+#   LONG_MIN_ROW_BYTES in all, twice that for several modules, which share a
+#   tile's x.  Below 4096 tokens: wide outputs (2048 -> 14336 rank 64, 2560 tokens
+#   64% of the time; 4096 -> 1024 rank 40, 4096 tokens 15.0 / 20.3, rank 64 17.0 /
+#   20.8; 8192 -> 512 rank 40, 2560 tokens 20.9 / 28.4) or, of the highest ranks, a
+#   K that one round of the fused kernel is slow over (14336 -> 1024 rank 64, 2048
+#   tokens 42.5 / 32.7).  Beyond: any but narrow outputs of a short K (4096 ->
+#   512 rank 40, 5120 tokens 9% slower; fp32: any).
+#   fp32: 4096 -> 1024 rank 64, 4096 tokens 37.1 / 45.5, 8192 tokens 79.5 / 73.6;
+#   768 -> 3072 rank 64, 4096 tokens 35.5 / 30.9, 8192 tokens 76.9 / 52.2.
+# * Above rank 64 the other choice is the split pair, slower from
+#   LONG_MIN_TOKENS on in 16 bits (64 -> 64 rank 72, 2048 tokens 7.6 / 7.1; 1024 ->
+#   1024 rank 128, 4096 tokens 18.0 / 13.2; 4096 -> 4096 rank 128, 1024 tokens 19.3 /
+#   21.5, 2048 tokens 33.3 / 28.8; of 144 sizes only 64 -> 4096 rank 72, 2048 tokens
+#   the other way, 12.7 / 13.4), and the faster one in fp32 (rank 128, 4200 of 5600
+#   tokens, 4096 -> 4096 114 / 135 us, 14336 -> 4096 280 / 334; rank 96, 1024 ->
+#   4096 58 / 69).  Through MultiLoraLinear, where the split pair's shrink runs
+#   beside the base GEMM: 4096 -> 4096 rank 128, 2048 tokens 107 / 85, 16384 tokens
+#   522 / 469; 4096 -> 2 x 14336 rank 256, 4096 tokens 1004 / 889; no size slower.
 LONG_MAX_RANK = 256  # half of it in fp32
 LONG_MIN_Y_BYTES = 112 << 20
 LONG_MIN_BYTES = 40 << 20
 LONG_MIN_ROW_BYTES = 8192
 LONG_MIN_TOKENS = 2048
+FUSED_ROUND_TOKENS = 4096
 
 
 def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules: int = 1) -> bool:
@@ -549,10 +572,44 @@ def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules:
         return es == 2 and rank <= LONG_MAX_RANK and tokens >= LONG_MIN_TOKENS
     if in_features > FUSED_MAX_K or not _long_grid_fits(tokens, es, rank, out_features, modules):
         return False
-    if rank <= 32:
-        return 2 * es * tokens * out_features >= LONG_MIN_Y_BYTES
-    return (es * (in_features + out_features) >= LONG_MIN_ROW_BYTES
-            and es * tokens * (in_features + 2 * out_features) >= LONG_MIN_BYTES * min(modules, 2))
+    pays = _long_pays_to_rank_32 if rank <= 32 else _long_pays_above_rank_32
+    return pays(tokens, es, rank, in_features, out_features, modules)
+
+
+def _long_pays_to_rank_32(tokens: int, es: int, rank: int, K: int, N: int, modules: int) -> bool:
+    y = 2 * es * tokens * N
+    if y < LONG_MIN_Y_BYTES:
+        return False
+    if tokens <= FUSED_ROUND_TOKENS:
+        if modules > 1:
+            return rank > 16 or N >= 4 * K or N >= 12288
+        return tokens > FUSED_ROUND_TOKENS // 2 and (N >= 2 * K or (es == 2 and rank > 16))
+    if es == 4:
+        if 768 < N < 3072 and (rank > 16 or K < 4096):
+            return y >= (320 if rank > 16 else 448) << 20
+    elif rank <= 16:
+        if 512 < N // modules < 1536 and K <= 1024:
+            return y >= 448 << 20
+        if modules == 1 and 512 < N < 3072 and K <= 4 * N:
+            return y >= 224 << 20
+    return True
+
+
+def _long_pays_above_rank_32(tokens: int, es: int, rank: int, K: int, N: int, modules: int) -> bool:
+    if es * (K + N) < LONG_MIN_ROW_BYTES or es * tokens * (K + 2 * N) < LONG_MIN_BYTES * min(modules, 2):
+        return False
+    if modules > 1:
+        return True
+    top = rank > 48  # four rank tiles in the fused kernel
+    if tokens > FUSED_ROUND_TOKENS:
+        return es == 4 or N >= 2048 or K + N >= 5120 or (K >= 4096 and top) or tokens >= 2 * FUSED_ROUND_TOKENS
+    if es == 4:
+        wide = N >= 2 * K or (N >= 4096 and N > K)
+    else:
+        wide = N >= 8192 or (N >= 4096 and (top or (tokens > FUSED_ROUND_TOKENS // 2 and K <= 1024)))
+    if wide and tokens > 1024:
+        return True
+    return es == 2 and top and tokens <= FUSED_ROUND_TOKENS // 2 and K >= 8192
 
 
 def _long_grid_fits(tokens: int, es: int, rank: int, out_features: int, modules: int) -> bool:

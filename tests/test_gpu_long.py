@@ -152,7 +152,7 @@ def test_long_and_fused_paths_give_the_same_bits(gpu, dtype, rows, row_len, K, N
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
 @pytest.mark.parametrize("rank", [16, 64])
 def test_a_linear_alone_and_with_its_siblings_gives_the_same_bits(gpu, monkeypatch, dtype, rank):
-    """Sizes for which a Linear alone takes the fused kernel and with its siblings the long path (the first forward
+    """A rule by which a Linear alone takes the fused kernel and with its siblings the long path (the first forward
     runs Linears alone, later ones the learned siblings together): equal outputs, and both kernels really ran."""
     ran = []
     calls = sgmv._native.calls()
@@ -166,11 +166,8 @@ def test_a_linear_alone_and_with_its_siblings_gives_the_same_bits(gpu, monkeypat
     monkeypatch.setattr(sgmv._native, "calls", lambda: spy)
     g = torch.Generator().manual_seed(rank)
     K, shapes, tokens = 1000, {"q": 1536, "k": 264, "v": 264}, 1200
-    es = torch.empty((), dtype=dtype).element_size()
-    # thresholds between k or v alone and q alone or all together
-    monkeypatch.setattr(sgmv, "LONG_MIN_Y_BYTES", 2 * es * tokens * 1000)
-    monkeypatch.setattr(sgmv, "LONG_MIN_BYTES", es * tokens * 2500)
-    monkeypatch.setattr(sgmv, "LONG_MIN_ROW_BYTES", 0)
+    # a line between k or v alone and q alone or all together
+    monkeypatch.setattr(sgmv, "long_ok", lambda plan, cache, fin, fout, modules=1: fout >= 1000)
     adapters = {f"a{i}": {m: peft_layer(g, K, n, r, 2.0 * r) for m, n in shapes.items()} for i, r in enumerate([rank, 5])}
     cache = make_cache(adapters, {m: (K, n) for m, n in shapes.items()}, 2, rank, gpu, dtype)
     slots = cache.ensure_resident(["a0", "a1", "a0"])

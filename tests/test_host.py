@@ -615,8 +615,17 @@ def test_long_workspace_size_is_64_bit():
 @pytest.mark.parametrize("rank,tokens,fin,fout,modules,want", [
     (16, 8192, 4096, 4096, 1, True), (16, 4096, 4096, 4096, 1, False), (32, 1024, 4096, 28672, 2, True),
     (64, 2048, 4096, 4096, 1, True), (64, 1024, 4096, 4096, 1, False), (64, 16384, 1024, 1024, 1, False),
-    (64, 3980, 2048, 3072, 3, False), (64, 3980, 2048, 3072, 1, True), (64, 8192, 20480, 4096, 1, False),
-    (72, 2048, 64, 64, 1, True), (72, 2047, 64, 64, 1, False), (264, 4096, 64, 64, 1, False)])
+    # 2048 -> 3072 takes 20.0 to 22.9 us by either path up to 4096 tokens, 5 to 9% more by the long one
+    (64, 3980, 2048, 3072, 3, False), (64, 3980, 2048, 3072, 1, False), (64, 8192, 20480, 4096, 1, False),
+    (72, 2048, 64, 64, 1, True), (72, 2047, 64, 64, 1, False), (264, 4096, 64, 64, 1, False),
+    # up to 4096 tokens: wide outputs, or the highest ranks over a long K
+    (40, 4096, 4096, 1024, 1, False), (64, 3072, 8192, 512, 1, False), (40, 2560, 2048, 14336, 1, True),
+    (64, 2048, 14336, 1024, 1, True), (40, 2048, 14336, 1024, 1, False), (16, 2048, 14336, 14336, 1, False),
+    (16, 3584, 3072, 8192, 1, True), (8, 4096, 3072, 9216, 3, False),
+    # beyond: not narrow outputs of a short K, nor middling outputs of low rank before twice or four times the bytes
+    (40, 5120, 4096, 512, 1, False), (64, 5120, 4096, 512, 1, True), (40, 9000, 4096, 512, 1, True),
+    (8, 14336, 2048, 2048, 1, False), (8, 28672, 2048, 2048, 1, True), (32, 14336, 2048, 2048, 1, True),
+    (8, 14336, 768, 2304, 3, False), (8, 65536, 768, 2304, 3, True)])
 def test_long_path_rule(rank, tokens, fin, fout, modules, want):
     """Which long-segment calls take the two-launch path (bf16, one adapter); never short segments."""
     from types import SimpleNamespace as Obj
@@ -627,6 +636,18 @@ def test_long_path_rule(rank, tokens, fin, fout, modules, want):
     assert sgmv.long_ok(Obj(distinct_slots=1, tokens_cap=tokens), cache, fin, fout, modules) == want
     assert not sgmv.long_ok(Obj(distinct_slots=None, tokens_cap=tokens), cache, fin, fout, modules)
     assert not sgmv.long_ok(Obj(distinct_slots=tokens // 32, tokens_cap=tokens), cache, fin, fout, modules)
+
+
+@pytest.mark.parametrize("rank,tokens,fin,fout,want", [
+    (64, 4096, 4096, 1024, False), (64, 8192, 4096, 1024, True), (64, 4096, 768, 3072, True), (64, 2048, 3072, 768, False),
+    (16, 6656, 768, 3072, True), (8, 4096, 768, 3072, False), (8, 14336, 2048, 2048, False), (32, 20480, 2048, 2048, True)])
+def test_long_path_rule_in_fp32(rank, tokens, fin, fout, want):
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    cache = Obj(rank8_cap=rank, dtype=torch.float32)
+    assert sgmv.long_ok(Obj(distinct_slots=1, tokens_cap=tokens), cache, fin, fout) == want
 
 
 @pytest.mark.parametrize("rank", [65, 96, 128, 256])
