@@ -652,6 +652,41 @@ class StackedFusedLaunch:
         self.n.check(self.lib.pl_lora_fused_stacked(*self.args), "pl_lora_fused_stacked")
 
 
+class LongLaunch:
+    """Long segments of one or several Linears fed the same x: the two launches of pl_lora_long_stacked.
+
+    `workspaces` (one per module, tokens_cap x the padded rank) may serve many launches of one stream."""
+
+    def __init__(self, x, ys, cache, modules, plan, workspaces):
+        import ctypes
+
+        from polylora_amd import _native
+
+        self.lib, self.n = _native.load(), _native
+        n = len(modules)
+        self.mods = (ctypes.c_int32 * n)(*(cache.module_index[m] for m in modules))
+        self.yptrs = (ctypes.c_void_p * n)(*(y.data_ptr() for y in ys))
+        self.ldys = (ctypes.c_int64 * n)(*(y.stride(0) for y in ys))
+        self.Ns = (ctypes.c_int32 * n)(*(int(y.shape[1]) for y in ys))
+        self.ws = (ctypes.c_void_p * n)(*(w.data_ptr() for w in workspaces[:n]))
+        self.args = (_native.dtype_code(x.dtype), x.data_ptr(), x.stride(0), int(x.shape[1]), n, self.mods,
+                     self.yptrs, self.ldys, self.Ns, cache.arena.data_ptr(), cache.table.data_ptr(),
+                     len(cache.module_index), cache.rank8_cap, plan.tok.data_ptr(), plan.groups.data_ptr(),
+                     plan.meta.data_ptr(), max(1, plan.group_cap), plan.group_tokens, plan.tokens_cap, self.ws,
+                     workspaces[0].numel(), _native.PL_EPI_FALLBACK, torch.cuda.current_stream().cuda_stream)
+        self.keep = (x, ys, plan, workspaces)
+
+    @staticmethod
+    def workspaces(cache, plan) -> list:
+        from polylora_amd import _native
+
+        nbytes = _native.load().pl_lora_long_workspace_bytes(_native.dtype_code(cache.dtype), plan.tokens_cap, cache.rank8_cap)
+        return [torch.empty(int(nbytes), dtype=torch.uint8, device=cache.device) for _ in range(_native.PL_MAX_STACKED_MODULES)]
+
+    def __call__(self):
+        self.n.check(self.lib.pl_lora_long_stacked(*self.args), "pl_lora_long_stacked")
+
+
 def time_launches(fns: list, reps: int, warmup: int = 2) -> float:
     """Milliseconds per pass over `fns`, launched back to back on the current stream between two events."""
     stream = torch.cuda.current_stream()
@@ -990,7 +1025,7 @@ class LaunchEntry:
     """One launch of a forward's LoRA sequence: what it serves and how to issue it."""
 
     label: str  # launch type, e.g. "q/k/v stacked shrink"
-    part: str  # "shrink", "expand" or "fused"
+    part: str  # "shrink", "expand", "fused", "long shrink" (issues the expand as well) or "long expand"
     modules: list  # wrapped Linear names served
     fn: object  # issues the launch
     owner: object  # the launch object (shared by a shrink and its expand)
@@ -1005,7 +1040,8 @@ def forward_launch_sequence(pm, plan, xs: dict, T: int, gen) -> list:
     Sibling Linears that read the same input (q/k/v, gate/up) share one
     stacked launch, as MultiLoraLinear does once it has seen a forward.  Where
     the plan suits the fused kernel each set takes one pl_lora_fused(_stacked)
-    launch; decode-sized batches one pl_lora_decode_stacked launch (split
+    launch, or the two of pl_lora_long_stacked where the forward does (two
+    entries, the first of which issues both); decode-sized batches one pl_lora_decode_stacked launch (split
     shrink and expand with the hand-off inside the launch); otherwise one
     stacked shrink and one stacked expand.  Every module type writes its own
     y, so siblings in one launch never share an output.
@@ -1020,7 +1056,7 @@ def forward_launch_sequence(pm, plan, xs: dict, T: int, gen) -> list:
         leaf = s.name.rsplit(".", 1)[-1]
         if leaf not in leaf_ys:
             leaf_ys[leaf] = torch.randn(T, s.out_features, generator=gen, device=device, dtype=torch.bfloat16)
-    out = []
+    out, workspaces = [], None
     for s in pm.module_specs:
         parent, leaf = s.name.rsplit(".", 1)
         if leaf in ("k_proj", "v_proj", "up_proj"):
@@ -1031,6 +1067,14 @@ def forward_launch_sequence(pm, plan, xs: dict, T: int, gen) -> list:
         tag += " stacked" if len(names) > 1 else ""
         k = by_name[names[0]].in_features
         outs = [leaf_ys[n.rsplit(".", 1)[-1]] for n in names]
+        high = cache.rank8_cap > sgmv.FUSED_MAX_RANK and sgmv.long_ok(plan, cache, k, outs[0].shape[1])
+        if high or (sgmv.fused_ok(plan, cache, k)
+                    and all(sgmv._use_long(xs[k], plan, cache, [y.shape[1] for y in outs], None))):
+            workspaces = workspaces or LongLaunch.workspaces(cache, plan)
+            g = LongLaunch(xs[k], outs, cache, names, plan, workspaces)
+            out += [LaunchEntry(f"{tag} long shrink", "long shrink", names, g, g),
+                    LaunchEntry(f"{tag} long expand", "long expand", names, lambda: None, g)]
+            continue
         if sgmv.fused_ok(plan, cache, k):
             f = (FusedLaunch(xs[k], outs[0], cache, names[0], plan) if len(names) == 1
                  else StackedFusedLaunch(xs[k], outs, cache, names, plan))
@@ -1060,10 +1104,10 @@ def launch_bytes(pm, modules: list, part: str, adapter_ids: list, lens: list) ->
     uniq = sorted({a for a, _ in rows})
     k = specs[modules[0]].in_features
     total = 0
-    if part in ("shrink", "fused"):
+    if part in ("shrink", "fused", "long shrink"):
         total += 2 * k * sum(n for a, n in rows if any(_rank_of(pm, a, m) > 0 for m in modules))
         total += sum(2 * _rank_of(pm, a, m) * k for m in modules for a in uniq)
-    if part in ("expand", "fused"):
+    if part in ("expand", "fused", "long expand"):
         for m in modules:
             nout = specs[m].out_features
             total += 4 * nout * sum(n for a, n in rows if _rank_of(pm, a, m) > 0)
@@ -1095,14 +1139,17 @@ def time_lora_ops(pm, adapter_ids: list, tokens_per_row: int, seq_lens: torch.Te
     lens = [min(int(v), tokens_per_row) for v in seq_lens.cpu().tolist()]
     seq_bytes = sum(launch_bytes(pm, e.modules, e.part, adapter_ids, lens) for e in entries)
     seq = [e.fn for e in entries]
-    stacks = list({id(e.owner): e.owner for e in entries if e.part != "fused"}.values())
+    stacks = list({id(e.owner): e.owner for e in entries if e.part in ("shrink", "expand")}.values())
     fused = [e.fn for e in entries if e.part == "fused"]
+    long = [e.fn for e in entries if e.part == "long shrink"]
     total_ms = time_launches(seq, reps)
     sh_ms = time_launches([st.shrink for st in stacks], reps) if stacks else 0.0
     ex_ms = time_launches([st.expand for st in stacks], reps) if stacks else 0.0
     fu_ms = time_launches(fused, reps) if fused else 0.0
-    return {"pairs_ms": total_ms, "shrink_ms": sh_ms, "expand_ms": ex_ms, "fused_ms": fu_ms, "per_type_us": per_type,
-            "group_tokens": plan.group_tokens, "launches": len(seq), "fused_launches": len(fused), "bytes": seq_bytes}
+    lo_ms = time_launches(long, reps) if long else 0.0
+    return {"pairs_ms": total_ms, "shrink_ms": sh_ms, "expand_ms": ex_ms, "fused_ms": fu_ms, "long_ms": lo_ms,
+            "per_type_us": per_type, "group_tokens": plan.group_tokens, "launches": len(seq),
+            "fused_launches": len(fused), "long_launches": 2 * len(long), "bytes": seq_bytes}
 
 
 def cpu_baseline_layer(pm, adapter_ids: list, budget_s: float, lens: list | None = None, seq: int = 1,
@@ -1547,13 +1594,16 @@ def run_prefill(args, pm) -> dict:
         out["lora_kernels_gbs_x_per_module"] = round(nb["total"] / (kern_ms * 1e-3) / 1e9, 1)
         out["lora_kernels_mfma_tflops"] = round(nb["flops"] / (kern_ms * 1e-3) / 1e12, 2)
         out["lora_kernels_pct_mfma_bf16"] = round(100 * nb["flops"] / (kern_ms * 1e-3) / 1e12 / MFMA_BF16_PEAK_TFLOPS, 3)
-        out["roofline"] = sequence_roofline("one prefill forward's LoRA launches (pl_lora_fused_tile)",
+        out["roofline"] = sequence_roofline("one prefill forward's LoRA launches (pl_long_shrink and pl_long_expand, "
+                                            "pl_lora_fused_tile)",
                                             nb["shared_x"], kern_ms, kt["launches"], "prefill")
         out["lora_kernels_shrink_ms"] = round(kt["shrink_ms"], 3)
         out["lora_kernels_expand_ms"] = round(kt["expand_ms"], 3)
         out["lora_kernels_fused_ms"] = round(kt["fused_ms"], 3)
+        out["lora_kernels_long_ms"] = round(kt["long_ms"], 3)
         out["lora_kernel_launches"] = kt["launches"]
         out["lora_fused_launches"] = kt["fused_launches"]
+        out["lora_long_launches"] = kt["long_launches"]
 
         def base_fwd():
             return pm.base_model(input_ids=ids, use_cache=False).last_hidden_state
@@ -1733,7 +1783,7 @@ def run_churn(args) -> dict:
 
 # ----------------------------------------------------------------------------- main
 # ----------------------------------------------------------------------------- launch profiles
-SEQUENCE_KERNELS = ("pl_shrink", "pl_expand", "pl_lora_fused", "pl_decode_fused", "pl_refop", "pl_plan")
+SEQUENCE_KERNELS = ("pl_shrink", "pl_expand", "pl_lora_fused", "pl_long", "pl_decode_fused", "pl_refop", "pl_plan")
 PLAN_KERNEL = "pl_plan_kernel"
 COPY_KERNEL = "__amd_rocclr_copyBuffer"
 

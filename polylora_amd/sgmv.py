@@ -627,7 +627,7 @@ def _use_long(x: torch.Tensor, plan: SgmvPlan, cache, widths, stream: int | None
     two paths do, so modules that share x decide together; in fp32, where the
     long path's sums are the more exact, each decides as it does alone.
     """
-    if stream not in (None, _stream(x.device)):
+    if stream is not None and stream != _stream(x.device):
         return [False] * len(widths)
     if x.element_size() == 2:
         return [long_ok(plan, cache, x.shape[1], sum(widths), len(widths))] * len(widths)

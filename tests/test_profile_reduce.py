@@ -150,3 +150,46 @@ def test_reduce_graph_trace_splits_bursts_and_compares_steps(tmp_path, capsys):
     # a trace without the four bursts is refused
     _write(tmp_path / "short.csv", TRACE_COLS, rows[:4])
     assert bench.main(["--reduce-graph-trace", "--trace", str(tmp_path / "short.csv"), "--profile-passes", "5"]) == 1
+
+
+@pytest.mark.parametrize("rank,takes_long,want", [
+    # (part, modules) of each entry: q/k/v with their summed width, o alone
+    (16, lambda fout: fout > 64, ["long shrink 3", "long expand 3", "fused 1"]),
+    (16, lambda fout: False, ["fused 3", "fused 1"]),
+    (128, lambda fout: True, ["long shrink 3", "long expand 3", "long shrink 1", "long expand 1"]),
+    (128, lambda fout: False, ["shrink 3", "expand 3", "shrink 1", "expand 1"])])
+def test_launch_sequence_takes_the_long_path_where_the_forward_does(monkeypatch, rank, takes_long, want):
+    """bench.forward_launch_sequence issues what MultiLoraLinear runs for long segments: the two-launch path where
+    sgmv's rule says so, each set's two dispatches as two entries whose bytes are the set's bytes together."""
+    from types import SimpleNamespace as Obj
+
+    import torch
+
+    from polylora_amd import sgmv
+
+    monkeypatch.setattr(sgmv, "long_ok", lambda plan, cache, fin, fout, modules=1: takes_long(fout))
+
+    class Launch:
+        def __init__(self, x, y, cache, names, plan, *rest):
+            self.shrink = self.expand = lambda: None
+
+        def __call__(self):
+            pass
+
+        workspaces = staticmethod(lambda cache, plan: ["ws"])
+
+    for name in ("FusedLaunch", "StackedFusedLaunch", "StackedLaunch", "DecodeLaunch", "LongLaunch"):
+        monkeypatch.setattr(bench, name, Launch)
+    specs = [Obj(name=f"l.0.{leaf}_proj", in_features=32, out_features=n) for leaf, n in (("q", 32), ("k", 24), ("v", 24), ("o", 32))]
+    cache = Obj(device=torch.device("cpu"), rank8_cap=rank, dtype=torch.bfloat16, decode_handoff=True,
+                ranks=None, module_index={s.name: i for i, s in enumerate(specs)})
+    pm = Obj(adapter_cache=cache, module_specs=specs, config=Obj(base_adapter_id="__base__"))
+    T = 4096
+    plan = Obj(distinct_slots=1, tokens_cap=T, group_tokens=16)
+    entries = bench.forward_launch_sequence(pm, plan, {32: torch.zeros(T, 32, dtype=torch.bfloat16)}, T,
+                                            torch.Generator().manual_seed(0))
+    assert [f"{e.part} {len(e.modules)}" for e in entries] == want
+    monkeypatch.setattr(bench, "_rank_of", lambda pm, a, m: rank)
+    total = sum(bench.launch_bytes(pm, e.modules, e.part, ["a"], [T]) for e in entries)
+    whole = sum(bench.launch_bytes(pm, m, "fused", ["a"], [T]) for m in (["l.0.q_proj", "l.0.k_proj", "l.0.v_proj"], ["l.0.o_proj"]))
+    assert total == whole > 0
