@@ -18,7 +18,6 @@ There is no CPU path: CPU tensors raise.
 
 from __future__ import annotations
 
-import ctypes
 from collections import deque
 
 import torch
@@ -685,31 +684,15 @@ def lora_fused(
 def _cache_args(cache, module_name: str) -> tuple:
     """(arena, table, module count, table column, rank capacity) of a module as pl_lora_fused takes them.
 
-    The arena and table are allocated once with the cache, so the tuple is
-    built once per cache and module.
+    Built once per cache and module, in a memo that the cache drops whenever
+    it allocates a new arena and table (GpuAdapterCache.to), so it cannot
+    outlive the memory it points at.
     """
     args = cache.__dict__.setdefault("_launch_args", {})
     hit = args.get(module_name)
     if hit is None:
         hit = args[module_name] = (cache.arena.data_ptr(), cache.table.data_ptr(), len(cache.module_index),
                                    cache.module_index[module_name], cache.rank8_cap)
-    return hit
-
-
-def _cache_args_c(cache, module_name: str) -> tuple:
-    """_cache_args as ctypes objects, built once per cache and module.
-
-    Kept in the same memo as _cache_args, which the cache drops whenever it
-    allocates a new arena and table (GpuAdapterCache.to), so neither form
-    can outlive the memory it points at.
-    """
-    args = cache.__dict__.setdefault("_launch_args", {})
-    key = ("ctypes", module_name)
-    hit = args.get(key)
-    if hit is None:
-        arena, table, n_modules, column, ldt = _cache_args(cache, module_name)
-        hit = args[key] = (ctypes.c_void_p(arena), ctypes.c_void_p(table), ctypes.c_int32(n_modules),
-                           ctypes.c_int32(column), ctypes.c_int32(ldt))
     return hit
 
 
