@@ -1,10 +1,11 @@
 """The two-launch path of long segments (lora_long_stacked) at the edges of its tiles, against the oracle.
 
-Segments around one, two and four 16-token tiles, so that a unit of tiles
-holds one slot or several; K around one wave's step and a turn of the four
-waves; N around an MFMA tile and a workgroup's chunk; ranks around a pass (and
-two passes, above 64); a second module that some adapters do not have; plans
-of 16- and 64-token groups, and one with enough tiles for the two-tile shrink.
+Segments around one, two and four 16-token tiles; K around one wave's step and
+a turn of the four waves; N around an MFMA tile and a workgroup's chunk; ranks
+around a pass (and two passes, above 64); a second module that some adapters
+do not have; plans of 16- and 64-token groups, and one with enough tiles for
+the two-tile shrink.  Then units of two and four tiles of several slots, for
+launches large enough to have them; infinities and NaN; HIP graphs, streams.
 
 Reference: the fallback of layers.py:112-134 (reference_forward).
 """
@@ -74,6 +75,167 @@ def test_long_path_edges_match_the_oracle(gpu, dtype, group_tokens, rows, row_le
             keep = torch.tensor([[int(rk[s]) == 0 or m >= int(n) for m in range(row_len)]
                                  for s, n in zip(row_slot.tolist(), seq)])
             assert torch.equal(got[keep], base[keep])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize("ranks,Ns", [
+    ([32, 5, 17, 0, 16], (2048,)),  # expand units of two tiles
+    ([64, 33, 0, 8, 48], (2048,)),  # of four
+    ([128, 65, 40, 0, 9, 100], (2048,)),  # four, intermediates of up to 8 rank steps in fp32, 4 in 16 bits
+    ([256, 129, 70, 0, 40, 64], (2048,)),  # 8 rank steps in 16 bits; 64-rank shrink passes
+    ([64, 40, 0, 16], (1024, 256, 256, 512))])  # 64-rank shrink passes of four modules
+def test_units_of_several_slots_match_the_oracle(gpu, dtype, ranks, Ns):
+    """Many short segments of interleaved adapters, some without the modules, in launches large enough for shrink
+    units of two tiles and expand units of two or four: neighbouring tiles of a unit belong to different slots."""
+    print("case:", dtype, ranks, Ns, flush=True)
+    if dtype == torch.float32:
+        ranks = [min(r, sgmv.LONG_MAX_RANK // 2) for r in ranks]
+    rows, row_len, K, n_adapters = 220, 30, 72, 100
+    g = torch.Generator().manual_seed(sum(ranks) + len(Ns))
+    mods = [f"m{i}" for i in range(len(Ns))]
+    adapters = {}
+    for i in range(n_adapters):
+        r = ranks[i % len(ranks)]
+        adapters[f"a{i}"] = ({m: peft_layer(g, K, n, r, 2.0 * r) for m, n in zip(mods, Ns)} if r else
+                             {"other": peft_layer(g, 8, 8, 2, 4.0)})
+    shapes = dict({m: (K, n) for m, n in zip(mods, Ns)}, other=(8, 8))
+    cache = make_cache(adapters, shapes, n_adapters, max(ranks), gpu, dtype)
+    ids = list(adapters) + ["__base__"]
+    # every adapter first, so that all hold slots, then at random
+    pick = [ids[i] for i in range(n_adapters)] + [ids[i] for i in torch.randint(0, len(ids), (rows - n_adapters,), generator=g).tolist()]
+    row_slot = cache.ensure_resident(pick)
+    seq = torch.randint(0, row_len + 2, (rows,), generator=g, dtype=torch.int32)
+    plan = sgmv.SgmvPlan(row_slot, seq.to(gpu), row_len, cache.num_slots, distinct_slots=n_adapters, group_tokens=16)
+    # what the launch's choices look at: tiles, and workgroups of one-tile units
+    es = torch.empty((), dtype=dtype).element_size()
+    ldt, tiles = cache.rank8_cap, -(-plan.group_cap // 8) * 8
+    chunk = (512 if ldt * es > 128 else 1024) // es
+    assert tiles >= 512 and all(n * es % 128 == 0 for n in Ns)
+    assert tiles * sum(-(-n // chunk) for n in Ns) >= 2048
+    if len(Ns) == 4 or ldt == 256:
+        assert tiles // 2 * len(Ns) * -(-ldt // 32) >= 1536  # 64-rank passes
+    slots = plan.groups.cpu()[: int(plan.meta[3]), 0].view(-1, 8)  # [position on the XCD][XCD]
+    for unit in (2, 4):
+        several = sum(len(set(slots[i : i + unit, x].tolist())) > 1 for x in range(8) for i in range(0, slots.shape[0], unit))
+        assert several > slots.shape[0] // unit * 8 // 4, unit
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    bases = [torch.randn(rows, row_len, n, generator=g).to(dtype) for n in Ns]
+    got = [b.to(gpu).view(-1, b.shape[-1]) for b in bases]
+    sgmv.lora_long_stacked(x.to(gpu).view(-1, K), got, cache, mods, plan)
+    for m, y, base in zip(mods, got, bases):
+        A, B, rk, sc = oracle_slot_tensors(cache, adapters, m, dtype)
+        y = y.cpu().view(base.shape)
+        torch.testing.assert_close(y, reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc), **tol_for(dtype))
+        keep = torch.tensor([[int(rk[s]) == 0 or i >= int(n) for i in range(row_len)] for s, n in zip(row_slot.tolist(), seq)])
+        assert torch.equal(y[keep], base[keep])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("rank,N", [(5, 264), (40, 2048), (100, 264)])
+def test_infinities_and_nans_stay_in_their_tokens(gpu, dtype, rank, N):
+    """An infinity or NaN in x or in one adapter's weights gives the oracle's values, in its own tokens alone: rows of
+    a tile past its tokens, ranks past the slot's and K past the range are left out, not multiplied by zero."""
+    print("case:", dtype, rank, N, flush=True)
+    g = torch.Generator().manual_seed(rank)
+    rows, row_len, K = 40, 27, 72
+    adapters = {f"a{i}": {"m": peft_layer(g, K, N, max(1, rank - 2 * i), 2.0 * rank)} for i in range(3)}
+    adapters["a2"]["m"][0][0, 5] = float("inf")  # A of one adapter
+    cache = make_cache(adapters, {"m": (K, N)}, 3, rank, gpu, dtype)
+    row_slot = cache.ensure_resident([["a0", "a1", "a2", "__base__"][i % 4] for i in range(rows)])
+    seq = torch.randint(1, row_len + 1, (rows,), generator=g, dtype=torch.int32)
+    plan = sgmv.SgmvPlan(row_slot, seq.to(gpu), row_len, cache.num_slots, distinct_slots=3, group_tokens=16)
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    x[0, 0, 3], x[5, 0, K - 1], x[8, 0, 0] = float("inf"), float("nan"), float("-inf")
+    x[4, int(seq[4]) - 1, K - 1] = float("inf")  # the last token of a row, last of its slot's tile or not
+    x[9, :, :][int(seq[9]):] = float("nan")  # padding positions
+    base = torch.randn(rows, row_len, N, generator=g).to(dtype)
+    y = base.to(gpu).view(-1, N)
+    sgmv.lora_long_stacked(x.to(gpu).view(-1, K), [y], cache, ["m"], plan)
+    A, B, rk, sc = oracle_slot_tensors(cache, adapters, "m", dtype)
+    want = reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc)
+    got = y.cpu().view(base.shape)
+    assert bool(want.isnan().any()) and bool(want.isfinite().any())
+    assert torch.equal(got.isfinite(), want.isfinite())
+    ok = want.isfinite()
+    torch.testing.assert_close(got[ok], want[ok], **tol_for(dtype))
+
+
+def _long_case(gpu, seed, rank=24):
+    g = torch.Generator().manual_seed(seed)
+    K, shapes, tokens = 520, {"q": 1032, "k": 264}, 1300
+    adapters = {f"a{i}": {m: peft_layer(g, K, n, r, 2.0 * r) for m, n in shapes.items()} for i, r in enumerate([rank, 7])}
+    cache = make_cache(adapters, {m: (K, n) for m, n in shapes.items()}, 2, rank, gpu, torch.bfloat16)
+    slots = cache.ensure_resident(["a0", "a1", "__base__", "a0"])
+    plan = sgmv.SgmvPlan(slots, torch.tensor([325, 99, 200, 16], dtype=torch.int32, device=gpu), 325, cache.num_slots,
+                         distinct_slots=2)
+    x = torch.randn(tokens, K, generator=g).bfloat16().to(gpu)
+    bases = [torch.randn(tokens, n, generator=g).bfloat16().to(gpu) for n in shapes.values()]
+    return cache, list(shapes), plan, x, bases
+
+
+@pytest.mark.parametrize("rank", [24, 100])
+def test_long_path_in_a_graph(gpu, rank):
+    """Captured with its workspace (an allocation inside the capture), between other captured work; every replay,
+    with eager long calls between replays, equals the eager result."""
+    cache, mods, plan, x, bases = _long_case(gpu, 90 + rank, rank)
+    want = sgmv.lora_long_stacked(x, [b.clone() for b in bases], cache, mods, plan)
+    ys = [torch.empty_like(b) for b in bases]
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        for y, b in zip(ys, bases):
+            y.copy_(b)
+        sgmv.lora_long_stacked(x, ys[:1], cache, mods[:1], plan)
+        more = torch.ones(1 << 18, device=gpu)  # may take the first call's workspace
+        sgmv.lora_long_stacked(x, ys[1:], cache, mods[1:], plan)
+        more.add_(1.0)
+    for i in range(4):
+        for y in ys:
+            y.fill_(float(i))
+        eager = sgmv.lora_long_stacked(x, [b.clone() for b in bases], cache, mods, plan)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert all(torch.equal(a, b) for a, b in zip(ys, want)), i
+        assert all(torch.equal(a, b) for a, b in zip(eager, want)), i
+        assert bool((more == 2.0).all()), i
+
+
+def test_long_calls_on_two_streams(gpu):
+    """Calls that overlap on two streams have workspaces of their own: equal to the calls one after the other."""
+    cases = [_long_case(gpu, seed, rank) for seed, rank in ((101, 24), (102, 64))]
+    want = [sgmv.lora_long_stacked(x, [b.clone() for b in bases], cache, mods, plan) for cache, mods, plan, x, bases in cases]
+    streams = [torch.cuda.Stream() for _ in cases]
+    outs = [[[b.clone() for b in bases] for _ in range(20)] for *_, bases in cases]
+    torch.cuda.synchronize()
+    for i in range(20):
+        for (cache, mods, plan, x, _), s, ys in zip(cases, streams, outs):
+            with torch.cuda.stream(s):
+                sgmv.lora_long_stacked(x, ys[i], cache, mods, plan)
+    torch.cuda.synchronize()
+    for ys, ref in zip(outs, want):
+        for i, y in enumerate(ys):
+            assert all(torch.equal(a, b) for a, b in zip(y, ref)), i
+
+
+def test_a_stream_other_than_the_current_one_keeps_the_fused_kernel(gpu, monkeypatch):
+    """The workspace is allocated on the current stream, so lora_fused(stream=other) stays off the long path."""
+    cache, mods, plan, x, bases = _long_case(gpu, 103)
+    calls = []
+    launch = sgmv._long_launch
+    monkeypatch.setattr(sgmv, "_long_launch", lambda *a: (calls.append(1), launch(*a))[1])
+    monkeypatch.setattr(sgmv, "long_ok", lambda *a: True)
+    here = sgmv.lora_fused(x, bases[0].clone(), cache, mods[0], plan)
+    assert calls == [1]
+    both = sgmv.lora_fused_stacked(x, [b.clone() for b in bases], cache, mods, plan, stream=torch.cuda.current_stream().cuda_stream)
+    assert calls == [1, 1]
+    there, there2 = bases[0].clone(), [b.clone() for b in bases]
+    other = torch.cuda.Stream()
+    torch.cuda.synchronize()
+    sgmv.lora_fused(x, there, cache, mods[0], plan, stream=other.cuda_stream)
+    sgmv.lora_fused_stacked(x, there2, cache, mods, plan, stream=other.cuda_stream)
+    torch.cuda.synchronize()
+    assert calls == [1, 1]
+    assert torch.equal(here, there) and all(torch.equal(a, b) for a, b in zip(both, there2))
 
 
 def test_the_dispatch_takes_the_long_path_where_its_rule_says(gpu, monkeypatch):

@@ -127,3 +127,30 @@ def test_row_kernel_reads_x_before_an_overlapping_y(gpu, dtype, kind, rows, row_
         torch.testing.assert_close(y, want, **tol_for(dtype))
     else:
         assert torch.equal(y, want)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("K,N,rank", [(71, 65, 5), (1031, 1025, 16), (72, 264, 40)])
+def test_infinities_and_nans_stay_in_their_positions(gpu, dtype, K, N, rank):
+    """An infinity or NaN in x or in one adapter's weights gives the oracle's values, in its own positions alone."""
+    print("case:", dtype, K, N, rank, flush=True)
+    g = torch.Generator().manual_seed(K)
+    rows, row_len = 12, 21
+    adapters = {f"a{i}": {"m": peft_layer(g, K, N, max(1, rank - 2 * i), 2.0 * rank)} for i in range(3)}
+    adapters["a2"]["m"][0][0, 5] = float("inf")  # A of one adapter
+    cache = make_cache(adapters, {"m": (K, N)}, 3, rank, gpu, dtype, tiled=False)
+    row_slot = cache.ensure_resident([["a0", "a1", "a2", "__base__"][i % 4] for i in range(rows)])
+    seq = torch.randint(1, row_len + 1, (rows,), generator=g, dtype=torch.int32)
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    x[0, 0, 3], x[5, 0, K - 1], x[8, 0, 0] = float("inf"), float("nan"), float("-inf")
+    x[4, int(seq[4]) - 1, K - 1] = float("inf")
+    x[9, :, :][int(seq[9]):] = float("nan")  # padding positions
+    base = torch.randn(rows, row_len, N, generator=g).to(dtype)
+    y = base.to(gpu).view(-1, N)
+    sgmv.lora_apply_rows(x.to(gpu).view(-1, K), y, cache, "m", row_slot, seq.to(gpu), row_len)
+    A, B, rk, sc = oracle_slot_tensors(cache, adapters, "m", dtype)
+    want = reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc)
+    got = y.cpu().view(base.shape)
+    assert bool(want.isnan().any()) and torch.equal(got.isfinite(), want.isfinite())
+    ok = want.isfinite()
+    torch.testing.assert_close(got[ok], want[ok], **tol_for(dtype))
