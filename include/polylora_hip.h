@@ -352,8 +352,9 @@ int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, int32_t K, i
  * (any K, N, strides, alignment).  Writes y[b*row_len+m] for m < seq_len[b].
  * Rows whose slot is <= 0 or >= num_slots get no LoRA.  tmp is
  * [rows*row_len][ldt] fp32 scratch with ldt >= the largest rank (written
- * for ldt above 256, for more than 2^24 tiles of 16 positions and for a y
- * whose rows lie over other rows of x: else the intermediate stays on chip).
+ * for ldt above 256, for many rows of few positions and low ranks, for more
+ * than 2^24 tiles of 16 positions and for a y whose rows lie over other rows
+ * of x: else the intermediate stays on chip).
  * y may be x, or overlap it in any way: every x is read before its row, or
  * another that lies over it, is written. */
 int pl_lora_apply_rows(int32_t dtype, const void* x, int64_t ldx, int32_t K, void* y,

@@ -207,7 +207,7 @@ int pl_fused_phase(int mode, int32_t dtype, const void* x, int64_t ldx, int32_t 
 // The LoRA of rows straight from the row -> slot map and lengths, at any K, N,
 // stride and element alignment (sgmv_wide.hip), for rank capacities up to
 // kWideRankMax.  Returns PL_WIDE_DECLINED, having launched nothing, for what
-// it does not take.
+// it does not take or is slower at than the plain row kernels.
 constexpr int kWideRankMax = 256;
 constexpr int PL_WIDE_DECLINED = -101;
 int pl_wide_rows_launch(int32_t dtype, const void* x, int64_t ldx, int32_t K, void* y, int64_t ldy,

@@ -3,10 +3,12 @@
 // They serve two callers: the reference-layout operator API
 // (sgmv_lora_a_fwd / sgmv_lora_b_fwd, sgmv.py:141-175 and :278-328, weights
 // [slots][k][n] with arbitrary strides) where its MFMA path (sgmv_refop.hip)
-// declines the shape or gets no workspace, and, on the slot arena, rank
-// capacities above kWideRankMax (every other row call of the slot arena runs
-// the MFMA kernel of sgmv_wide.hip: 5 to 80 times as fast at 1 to 4096 rows).
-// Throughput is not their goal.
+// declines the shape or gets no workspace, and, on the slot arena, the row
+// calls that the MFMA kernel of sgmv_wide.hip declines: rank capacities above
+// kWideRankMax, many rows of few positions at low ranks, where these are the
+// faster ones (up to 6 times, 4096 rows of one position at rank 1), and a y
+// that lies over other rows of x.  Everywhere else that kernel is faster, up
+// to 80 times.
 //
 // Shrink: one wave per token row; lanes stride K, each rank column is a
 // wave-wide dot product finished with a butterfly reduction.

@@ -19,8 +19,11 @@
 // row -> slot map and the row lengths, with no plan and no scratch, at any K,
 // N, row stride and element alignment: 16-byte accesses at element alignment
 // (global memory allows them), and the elements past the last whole chunk of K
-// or N one by one.  Ranks go in passes of 16 * JT, up to kWideRankMax.
+// or N one by one.  Ranks go in passes of 16 * JT, up to kWideRankMax.  Many
+// rows of few positions at low ranks stay with the plain kernels
+// (plain_rows_faster).
 #include <algorithm>
+#include <cmath>
 
 #include "pl_common.h"
 
@@ -320,6 +323,25 @@ int row_overlap(const void* x, int64_t ldx, int64_t K, const void* y, int64_t ld
   return d > -ld && d < ld && d + N * es <= ld && d >= K * es - ld ? kOwnRow : kAcross;
 }
 
+// Whether the plain row kernels (a wave per row, a thread per output) are
+// the faster ones: with few positions per tile and low ranks the matrix cores
+// multiply padding, and a round of 16-wave workgroups costs 7 us whatever its
+// tiles hold.  Estimates of both in us, fitted to 2,370 sizes (1 to 16384
+// positions in rows of 1 to 1024, ranks 1 to 256, K and N 1 to 16384), where
+// the pick takes 1% more than the faster path on average and this kernel
+// alone took 16% more.  Plain / this kernel, bf16: 4096 rows of 1, 768 -> 768,
+// rank 1 17 / 66 us, rank 16 70 / 67; 4096 -> 4096, rank 1 76 / 154, rank 16 350 /
+// 154; fp32: 64 rows of 1, 4096 -> 4096, rank 1 13 / 24, rank 16 130 / 24.
+bool plain_rows_faster(int es, double T, double tiles, double per, double slices, double K, double N, double rank) {
+  const double k64 = std::ceil(K / 64) * 64, n256 = std::ceil(N / 256) * 256;
+  const double plain = 3 + 0.2 * rank + 1.2e-3 * rank * K +
+                       1e-6 * T * (rank * (0.14 * k64 + 0.39 * n256) + es * (0.05 * K + 1.36 * N));
+  const double r16 = std::max(rank, 16.0), f = es == 4 ? 1 : 0;
+  const double round = 1.2 + 5.4 * per + (1 + 2 * f) * 2.8e-5 * r16 * K + (1 + f) * 0.044 * per * r16;
+  const double wide = std::max(1.0, tiles * slices / 650) * round + 0.18e-6 * T * N * es;
+  return 1.1 * std::max(plain, 10.0) < wide;  // two launches: never under 10
+}
+
 template <int DT>
 void launch_wide_rows(const pl_wide_args& a, int32_t rank_cap, dim3 grid, hipStream_t s) {
   if (rank_cap <= 16)
@@ -353,6 +375,10 @@ int pl_wide_rows_launch(int32_t dtype, const void* x, int64_t ldx, int32_t K, vo
   a.cols = (int32_t)(per * step_cols);
   a.slices = (int32_t)((steps + per - 1) / per);
   if (!pl_grid_fits(pl_xcd_grid(tiles, a.slices), kWThreads)) return PL_WIDE_DECLINED;
+  if (pl_grid_fits((int64_t)rows * row_len * (((int64_t)N + 255) / 256), 256) &&  // the plain kernels' grid
+      plain_rows_faster(pl_elem_size(dtype), (double)rows * row_len, (double)tiles, (double)per, a.slices, K,
+                        N, rank_cap))
+    return PL_WIDE_DECLINED;
   a.x = x;
   a.ldx = ldx;
   a.K = K;

@@ -154,3 +154,31 @@ def test_infinities_and_nans_stay_in_their_positions(gpu, dtype, K, N, rank):
     assert bool(want.isnan().any()) and torch.equal(got.isfinite(), want.isfinite())
     ok = want.isfinite()
     torch.testing.assert_close(got[ok], want[ok], **tol_for(dtype))
+
+
+@pytest.mark.parametrize("dtype,rows,row_len,K,N,rank,plain", [
+    (torch.bfloat16, 4096, 1, 768, 768, 1, True), (torch.bfloat16, 4096, 1, 16, 16, 16, True),
+    (torch.bfloat16, 4096, 1, 768, 768, 64, False), (torch.bfloat16, 1024, 3, 100, 100, 2, True),
+    (torch.bfloat16, 64, 17, 1024, 1003, 4, False), (torch.float32, 256, 1, 4096, 1003, 1, True),
+    (torch.float32, 256, 1, 4096, 1003, 16, False), (torch.float32, 64, 1, 1000, 2000, 4, False)])
+def test_many_rows_of_low_rank_take_the_plain_kernels(gpu, dtype, rows, row_len, K, N, rank, plain):
+    """The row kernels' route, seen from the scratch (only the plain kernels write it), and the result on both."""
+    print("case:", dtype, rows, row_len, K, N, rank, flush=True)
+    g = torch.Generator().manual_seed(rows + K)
+    adapters = {"a": {"m": peft_layer(g, K, N, rank, 2.0 * rank)}}
+    cache = make_cache(adapters, {"m": (K, N)}, 1, rank, gpu, dtype, tiled=False)
+    row_slot = cache.ensure_resident([["a", "__base__"][i % 3 == 2] for i in range(rows)])
+    seq = torch.randint(1, row_len + 1, (rows,), generator=g, dtype=torch.int32)
+    x = torch.randn(rows, row_len, K, generator=g).to(dtype)
+    base = torch.randn(rows, row_len, N, generator=g).to(dtype)
+    dx, y, lens = x.to(gpu).view(-1, K), base.to(gpu).view(-1, N), seq.to(gpu)
+    tmp = torch.full((rows * row_len, rank), 12345.0, device=gpu)
+    arena, table, n_mod, column, _ = sgmv._cache_args(cache, "m")
+    rc = sgmv._native.calls().pl_lora_apply_rows(
+        sgmv._native.dtype_code(dtype), dx.data_ptr(), K, K, y.data_ptr(), N, N, arena, table, cache.num_slots, n_mod,
+        column, row_slot.data_ptr(), lens.data_ptr(), rows, row_len, tmp.data_ptr(), rank, 0, sgmv._stream(gpu))
+    sgmv._native.check(rc, "pl_lora_apply_rows")
+    assert bool((tmp != 12345.0).any()) == plain
+    A, B, rk, sc = oracle_slot_tensors(cache, adapters, "m", dtype)
+    want = reference_forward(x, base, seq, row_slot.cpu(), A, B, rk, sc)
+    torch.testing.assert_close(y.cpu().view(base.shape), want, **tol_for(dtype))
