@@ -268,7 +268,7 @@ def lora_apply(
         if fused_ok(plan, cache, int(x.shape[1])):
             _fused_launch(x, y, cache, module_name, plan, epilogue, None, _stream(x.device))
             return y
-        if long_ok(plan, cache, x.shape[1], y.shape[1]):
+        if long_ok(plan, cache, x.shape[1], y.shape[1]) and not _host_paces_pair(plan, cache, x.shape[1], y.shape[1]):
             _long_launch(x, [y], cache, [module_name], plan, epilogue, _stream(x.device))
             return y
         if _one_launch_ok(plan, cache, x.shape[1], y.shape[1]) and _own_rows(x, y):
@@ -609,6 +609,14 @@ def _long_pays_above_rank_32(tokens: int, es: int, rank: int, K: int, N: int, mo
     if wide and tokens > 1024:
         return True
     return es == 2 and top and tokens <= FUSED_ROUND_TOKENS // 2 and K >= 8192
+
+
+def _host_paces_pair(plan: SgmvPlan, cache, in_features: int, out_features: int) -> bool:
+    """Whether the split pair of a lora_apply above rank 64 needs less of the GPU than its call of the host: the long
+    path's takes 1 us more (calls back to back, 64 -> 64 rank 72, 2048 tokens 10.6 / 11.6 us, 4096 tokens 11.0 / 12.2;
+    256 -> 256 rank 128, 4096 tokens 10.8 / 11.9; 1024 -> 1024 rank 72, 2048 tokens 12.9 / 11.9)."""
+    return (FUSED_MAX_RANK < cache.rank8_cap <= 128 and plan.tokens_cap <= 4096
+            and cache.dtype.itemsize * plan.tokens_cap * (in_features + out_features) <= 4 << 20)
 
 
 def _long_grid_fits(tokens: int, es: int, rank: int, out_features: int, modules: int) -> bool:

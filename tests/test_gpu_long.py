@@ -244,7 +244,9 @@ def test_the_dispatch_takes_the_long_path_where_its_rule_says(gpu, monkeypatch):
     launch = sgmv._long_launch
     monkeypatch.setattr(sgmv, "_long_launch", lambda x, ys, *a: (calls.append(len(ys)), launch(x, ys, *a))[1])
     g = torch.Generator().manual_seed(5)
-    for rank, rows, n, want in ((16, 20, 1024, []), (16, 20, 17000, [1, 1]), (96, 20, 64, [1]), (96, 8, 64, [])):
+    # (rank 96, 64 outputs: a call that the host paces keeps the split pair)
+    for rank, rows, n, want in ((16, 20, 1024, []), (16, 20, 17000, [1, 1]), (96, 40, 64, [1]), (96, 20, 64, []),
+                                (96, 20, 2048, [1]), (96, 8, 2048, []), (160, 20, 64, [1])):
         adapters = {"a": {"m": peft_layer(g, 64, n, rank, 2.0 * rank)}}
         cache = make_cache(adapters, {"m": (64, n)}, 1, rank, gpu, torch.bfloat16)
         row_slot = cache.ensure_resident(["a"] * rows)
