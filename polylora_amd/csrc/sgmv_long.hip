@@ -47,7 +47,7 @@ struct pl_long_args {
   const void* x;
   int64_t ldx;
   int32_t K;
-  int32_t kw;        // shrink: K per wave, whole pairs of steps; 0: steps in turn
+  int32_t kw;        // shrink: K per wave, whole pairs of steps; 0: steps in turn (ranks above 64, fp32)
   const char* arena;
   const pl_slot_entry* table;
   int32_t num_modules;
@@ -133,7 +133,8 @@ constexpr int pl_long_shrink_lds() {
                                                                              : RT * JT * 1024);
 }
 
-template <int DT, int JT, int RT, int SB, bool XNT>
+// SHARE: the waves take shares of K (a.kw), else K steps in turn.
+template <int DT, int JT, int RT, int SB, bool XNT, bool SHARE>
 __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int job, int rb,
                                                    const pl_slot_entry& e,
                                                    const pl_long_tile (&tl)[RT],
@@ -220,12 +221,11 @@ __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int jo
         for (int cc = 0; cc < kCC; ++cc) acc[rt][jt] = pl_mfma_chunk_short<DT>(xm[cc], am[jt][cc], acc[rt][jt]);
     }
   };
-  // the waves take shares of K (a.kw) or K steps in turn; a step past the
-  // range loads only zeros
+  // a step past the range loads only zeros
   pl_u32x4 xa[2 * RT], aa[JT][kCC], xb[2 * RT], ab[JT][kCC];
-  const int next = a.kw > 0 ? kStep : kLWaves * kStep;
-  const int k1 = a.kw > 0 ? min(K, (wave + 1) * a.kw) : K;
-  int kb = wave * (a.kw > 0 ? a.kw : kStep);
+  constexpr int next = SHARE ? kStep : kLWaves * kStep;
+  const int k1 = SHARE ? min(K, (wave + 1) * a.kw) : K;
+  int kb = wave * (SHARE ? a.kw : kStep);
   load(xa, aa, kb);
   for (; kb + 2 * next < k1; kb += 2 * next) {
     load(xb, ab, kb + next);
@@ -279,7 +279,7 @@ __device__ __forceinline__ void pl_long_shrink_run(const pl_long_args& a, int jo
   }
 }
 
-template <int DT, int JT, int RT, bool XNT>
+template <int DT, int JT, int RT, bool XNT, bool SHARE>
 __global__ __launch_bounds__(64 * kLWaves, RT * JT <= 4 ? 3 : 2) void pl_long_shrink(pl_long_args a) {
   __shared__ __attribute__((aligned(16))) char smem[pl_long_shrink_lds<DT, JT, RT>()];
   const int xcd = (int)(blockIdx.x % kXcds);
@@ -324,11 +324,11 @@ __global__ __launch_bounds__(64 * kLWaves, RT * JT <= 4 ? 3 : 2) void pl_long_sh
     if (wrote) __syncthreads();  // the previous run's sums are read
     wrote = true;
     if (JT > 1 && e.rank - rb <= 16)
-      pl_long_shrink_run<DT, 1, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT>(a, job, rb, e, run, xt, smem);
+      pl_long_shrink_run<DT, 1, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT, SHARE>(a, job, rb, e, run, xt, smem);
     else if (JT > 2 && e.rank - rb <= 32)
-      pl_long_shrink_run<DT, JT < 2 ? JT : 2, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT>(a, job, rb, e, run, xt, smem);
+      pl_long_shrink_run<DT, JT < 2 ? JT : 2, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT, SHARE>(a, job, rb, e, run, xt, smem);
     else
-      pl_long_shrink_run<DT, JT, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT>(a, job, rb, e, run, xt, smem);
+      pl_long_shrink_run<DT, JT, RT, pl_long_stage_bytes<DT, JT, RT>(), XNT, SHARE>(a, job, rb, e, run, xt, smem);
   }
 }
 
@@ -579,14 +579,25 @@ int64_t long_units(const pl_long_args& a, int nt) {
   return (tiles + nt - 1) / nt;
 }
 
-template <int DT, int JT, int RT>
-void launch_shrink_rt(const pl_long_args& a, hipStream_t s) {
+template <int DT, int JT, int RT, bool SHARE>
+void launch_shrink_xnt(const pl_long_args& a, hipStream_t s) {
   const dim3 grid((unsigned)(long_units(a, RT) * kXcds * a.n_jobs * a.passes));
   // x is streamed only when one workgroup reads each of its rows
   if (a.n_jobs * a.passes == 1)
-    hipLaunchKernelGGL((pl_long_shrink<DT, JT, RT, true>), grid, dim3(64 * kLWaves), 0, s, a);
+    hipLaunchKernelGGL((pl_long_shrink<DT, JT, RT, true, SHARE>), grid, dim3(64 * kLWaves), 0, s, a);
   else
-    hipLaunchKernelGGL((pl_long_shrink<DT, JT, RT, false>), grid, dim3(64 * kLWaves), 0, s, a);
+    hipLaunchKernelGGL((pl_long_shrink<DT, JT, RT, false, SHARE>), grid, dim3(64 * kLWaves), 0, s, a);
+}
+
+template <int DT, int JT, int RT>
+void launch_shrink_rt(const pl_long_args& a, hipStream_t s) {
+  // shares in 16 bits up to rank 64 (one pass of 16 ranks at most: always)
+  if constexpr (DT == PL_F32)
+    launch_shrink_xnt<DT, JT, RT, false>(a, s);
+  else if constexpr (JT == 1)
+    launch_shrink_xnt<DT, JT, RT, true>(a, s);
+  else
+    a.kw > 0 ? launch_shrink_xnt<DT, JT, RT, true>(a, s) : launch_shrink_xnt<DT, JT, RT, false>(a, s);
 }
 
 template <int DT>
@@ -760,9 +771,11 @@ extern "C" int pl_lora_long_stacked(int32_t dtype, const void* x, int64_t ldx, i
   // In 16 bits the ranks of the fused kernel get its shares of K per wave, so
   // that each sum is the same additions in the same order and either kernel
   // gives the same bits: a Linear alone and with its siblings may take
-  // different ones.  (Steps in turn instead: 32768 tokens, 4096 -> 14336, rank
-  // 32 280.6 us, shares 279.5; 4096 tokens, 14336 -> 4096, rank 64 52.0 and 53.1;
-  // above rank 64 turns, 8192 tokens, 8192 -> 2048, rank 256 85.7 and 87.3.)
+  // different ones.  (Steps in turn instead: 32768 tokens, 4096 -> 14336, rank 32
+  // 280 us both; 4096 tokens, 14336 -> 4096, rank 64 52.1, shares 51.4; 16384
+  // tokens, 2048 -> 8192, rank 40 87.4 and 88.4; above rank 64, where the rule
+  // does not look at the outputs, turns: 8192 tokens, 8192 -> 2048, rank 256
+  // 84.8, shares 87.3.)
   const int64_t pair = 16 * E;
   const int64_t share = ((int64_t)K + kLWaves - 1) / kLWaves;
   a.kw = dtype != PL_F32 && ldt <= 64 ? (int32_t)((share + pair - 1) / pair * pair) : 0;
