@@ -504,7 +504,8 @@ class SgmvLaunch:
         self.stream = torch.cuda.current_stream()
         dt = _native.dtype_code(x.dtype)
         K, N = int(x.shape[1]), int(y.shape[1])
-        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype)
+        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
+                                                                                       plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = cache.rank8_cap
         gt = plan.group_tokens
@@ -540,7 +541,8 @@ class StackedLaunch:
         self.stream = torch.cuda.current_stream()
         dt = _native.dtype_code(x.dtype)
         K = int(x.shape[1])
-        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype)
+        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
+                                                                                       plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = cache.rank8_cap
         gt = plan.group_tokens
@@ -583,7 +585,8 @@ class DecodeLaunch:
         dt = _native.dtype_code(x.dtype)
         K = int(x.shape[1])
         n = len(modules)
-        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype)
+        splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
+                                                                                       plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = -(-cache.rank8_cap // 32) * 32
         gt = plan.group_tokens

@@ -181,22 +181,30 @@ def _workspace(device: torch.device, stream: int, position: int = 0) -> _Workspa
 # Small launches wait for one workgroup's chain of K steps instead: with few
 # groups, splits of 256 up to 4 of them (one decode launch, rank 64, 40 rows:
 # K = 1024 8.0 -> 6.0 us, K = 2048 9.5 -> 8.2; 256 rows over 64 adapters 9.0 ->
-# 7.0 and 15.0 -> 14.3), and with at most 16 groups splits of 512 up to 16
-# (8 rows, rank 64: K = 4096 8.6 -> 8.1, q/k/v 9.2 -> 8.9, K = 14336 12.1 -> 11.4;
-# at 24 groups and three modules it no longer pays: 8.9 -> 9.0).
+# 7.0 and 15.0 -> 14.3; of 180 sizes to 1000 rows the worst 9.9 -> 10.8).  With
+# at most 16 groups: splits of 512 up to 8 while every expand workgroup sums
+# the planes of few rows (rank 64: K = 4096, 8 rows 8.9 -> 8.1, gate/up, 24 rows
+# 11.8 -> 10.6; rank 16, gate/up, 48 rows 9.8 -> 12.9, so only to 32 rows), and
+# above K = 8192 one per 896, up to 16 (8 rows, rank 64: K = 14336 12.2 -> 11.5,
+# K = 11008 11.1 -> 10.6; K = 8192 with 16 is slower, 8192 -> 28672, rank 16, 12
+# rows 10.3 -> 13.4, q/k/v 9.2 -> 10.1).
 _K_PER_SPLIT = 1024
 _TARGET_SHRINK_BLOCKS = 2048
 _MAX_K_SPLITS = 8
 _FEW_GROUPS = 128
 _FEWEST_GROUPS = 16
+_FEW_TOKENS = 32
 
 
-def choose_k_splits(group_cap: int, K: int, dtype: torch.dtype) -> int:
-    """K splits of the shrink: about one per 1024 of K (at most 8), more for few groups, fewer when the group count
-    alone fills the GPU."""
+def choose_k_splits(group_cap: int, K: int, dtype: torch.dtype, tokens: int = 1) -> int:
+    """K splits of the shrink: about one per 1024 of K (at most 8), more for few groups (and few `tokens`), fewer when
+    the group count alone fills the GPU."""
     by_k = min(_MAX_K_SPLITS, max(1, -(-K // _K_PER_SPLIT)))
     if group_cap <= _FEWEST_GROUPS:
-        by_k = max(by_k, min(2 * _MAX_K_SPLITS, K // 512))
+        if K > _MAX_K_SPLITS * _K_PER_SPLIT:
+            by_k = max(by_k, min(2 * _MAX_K_SPLITS, K // 896))
+        elif tokens <= _FEW_TOKENS:
+            by_k = max(by_k, min(_MAX_K_SPLITS, K // 512))
     if group_cap <= _FEW_GROUPS:
         by_k = max(by_k, min(4, K // 256))
     by_groups = max(1, -(-_TARGET_SHRINK_BLOCKS // max(1, group_cap)))
@@ -361,7 +369,7 @@ def _shrink_geometry(lib, dt: int, K: int, dtype: torch.dtype, plan: SgmvPlan, r
             # the extra splits of few groups do not pay for their planes above rank 64 (37 rows, 14336 -> 4096, rank
             # 128: 16 splits 15.1 to 16.0 us, 8 splits 15.0)
             cap = plan.group_cap if ldt <= FUSED_MAX_RANK else max(plan.group_cap, _FEW_GROUPS + 1)
-            splits = choose_k_splits(cap, K, dtype)
+            splits = choose_k_splits(cap, K, dtype, rows)
         else:
             splits = k_splits
         planes = int(lib.pl_shrink_planes(dt, K, splits, plan.group_tokens))

@@ -778,3 +778,14 @@ def test_rows_of_y_over_other_rows_of_x_are_seen():
                         assert own or not sgmv._own_rows(x, y), (xs, ys, K, N, off, swap)
                         if xs == ys:
                             assert own == sgmv._own_rows(x, y), (xs, ys, K, N, off, swap)
+
+
+@pytest.mark.parametrize("groups,K,tokens,want", [
+    (8, 4096, 1, 8), (16, 4096, 32, 8), (16, 4096, 33, 4), (16, 4096, 128, 4), (17, 4096, 8, 4), (16, 1024, 200, 4),
+    (16, 8192, 1, 8), (16, 8192, 64, 8), (16, 3072, 8, 6), (16, 3072, 40, 4), (8, 11008, 8, 12), (8, 14336, 8, 16),
+    (16, 14336, 128, 16), (17, 14336, 8, 8), (128, 2048, 256, 4), (129, 2048, 256, 2)])
+def test_k_splits_of_few_groups(groups, K, tokens, want):
+    """More splits only where their planes are summed for few rows or the K chain is the longest."""
+    from polylora_amd import sgmv
+
+    assert sgmv.choose_k_splits(groups, K, torch.bfloat16, tokens) == want
