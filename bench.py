@@ -505,7 +505,7 @@ class SgmvLaunch:
         dt = _native.dtype_code(x.dtype)
         K, N = int(x.shape[1]), int(y.shape[1])
         splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
-                                                                                       plan.tokens_cap)
+                                                                            plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = cache.rank8_cap
         gt = plan.group_tokens
@@ -542,7 +542,7 @@ class StackedLaunch:
         dt = _native.dtype_code(x.dtype)
         K = int(x.shape[1])
         splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
-                                                                                       plan.tokens_cap)
+                                                                            plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = cache.rank8_cap
         gt = plan.group_tokens
@@ -586,7 +586,7 @@ class DecodeLaunch:
         K = int(x.shape[1])
         n = len(modules)
         splits = k_splits if k_splits is not None else sgmv.choose_k_splits(plan.group_cap, K, x.dtype,
-                                                                                       plan.tokens_cap)
+                                                                            plan.tokens_cap)
         rows = max(1, plan.tokens_cap)
         ldt = -(-cache.rank8_cap // 32) * 32
         gt = plan.group_tokens

@@ -275,8 +275,11 @@ int pl_sgmv_expand_stacked(int32_t dtype, void* const* ws, int32_t ldt, int64_t 
  * the results of that call are undefined, and a shrink workgroup that
  * arrives after the wait gave up can leave its counter above zero, so the
  * caller must zero all counter_ints words (with no call in flight) before
- * the next call; otherwise the status word stays 0.  Every other argument
- * is as for pl_sgmv_shrink_stacked and pl_sgmv_expand_stacked. */
+ * the next call; otherwise the status word stays 0.  Where a row of a y[i]
+ * lies over a row of x that another group or module may still read, the call
+ * takes the two launches instead (the counters are then not used).  Every
+ * other argument is as for pl_sgmv_shrink_stacked and
+ * pl_sgmv_expand_stacked. */
 int pl_lora_decode_stacked(int32_t dtype, const void* x, int64_t ldx, int32_t K, const void* arena,
                            const pl_slot_entry* table, int32_t num_modules, int32_t n_modules,
                            const int32_t* modules, void* const* ws, const int32_t* tok,

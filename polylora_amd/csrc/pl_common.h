@@ -204,6 +204,23 @@ int pl_fused_phase(int mode, int32_t dtype, const void* x, int64_t ldx, int32_t 
                    int64_t group_cap, int32_t group_tokens, int32_t slices, int32_t epilogue,
                    void* stream);
 
+// How rows of y, which a launch writes, lie over the rows of x it reads (T
+// rows each): not at all, row t over row t of x alone, or otherwise.
+enum class pl_overlap { apart, own_row, across };
+inline pl_overlap pl_row_overlap(const void* x, int64_t ldx, int64_t K, const void* y, int64_t ldy,
+                                 int64_t N, int64_t T, int es) {
+  const int64_t d = (int64_t)(reinterpret_cast<uintptr_t>(y) - reinterpret_cast<uintptr_t>(x));
+  const int64_t xbytes = ((T - 1) * ldx + K) * es, ybytes = ((T - 1) * ldy + N) * es;
+  if (d >= xbytes || -d >= ybytes) return pl_overlap::apart;
+  if (T == 1) return pl_overlap::own_row;
+  const int64_t ld = ldx * es;
+  if (ldx != ldy || ldx < K || ldy < N) return pl_overlap::across;
+  const int64_t col = ((d % ld) + ld) % ld;  // where y's rows start between two rows of x
+  if (col >= K * es && col + N * es <= ld) return pl_overlap::apart;
+  return d > -ld && d < ld && d + N * es <= ld && d >= K * es - ld ? pl_overlap::own_row
+                                                                    : pl_overlap::across;
+}
+
 // The LoRA of rows straight from the row -> slot map and lengths, at any K, N,
 // stride and element alignment (sgmv_wide.hip), for rank capacities up to
 // kWideRankMax.  Returns PL_WIDE_DECLINED, having launched nothing, for what

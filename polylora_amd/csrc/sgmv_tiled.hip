@@ -1572,6 +1572,17 @@ extern "C" int pl_lora_decode_stacked(int32_t dtype, const void* x, int64_t ldx,
     pl_set_error("pl_lora_decode_stacked: grid too large");
     return PL_ERR_LIMIT;
   }
+  // An expand of one group runs beside the shrinks of others, and of the other
+  // modules: where a y row may lie over an x row that one of those still
+  // reads, two launches, the shrink's first (the same bits).
+  for (int j = 0; j < n_modules; ++j) {
+    const pl_overlap o = pl_row_overlap(x, ldx, K, y[j], ldy[j], N[j], tmp_rows, pl_elem_size(dtype));
+    if (o == pl_overlap::across || (o == pl_overlap::own_row && n_modules > 1)) {
+      st = dispatch_shrink(dtype, sa, group_cap, reinterpret_cast<hipStream_t>(stream));
+      if (st) return st;
+      return dispatch_expand(dtype, ea, group_cap, reinterpret_cast<hipStream_t>(stream));
+    }
+  }
   pl_handoff h;
   h.counters = counters;
   h.n_shrink = (int32_t)n_shrink;

@@ -308,21 +308,6 @@ __global__ __launch_bounds__(kWThreads) void pl_lora_wide_rows(pl_wide_args a) {
   }
 }
 
-// How rows of y, which the launch writes, lie over the rows of x it reads
-// (T rows each): not at all, row t over row t of x alone, or otherwise.
-enum { kApart, kOwnRow, kAcross };
-int row_overlap(const void* x, int64_t ldx, int64_t K, const void* y, int64_t ldy, int64_t N, int64_t T, int es) {
-  const int64_t d = (int64_t)(reinterpret_cast<uintptr_t>(y) - reinterpret_cast<uintptr_t>(x));
-  const int64_t xbytes = ((T - 1) * ldx + K) * es, ybytes = ((T - 1) * ldy + N) * es;
-  if (d >= xbytes || -d >= ybytes) return kApart;
-  if (T == 1) return kOwnRow;
-  const int64_t ld = ldx * es;
-  if (ldx != ldy || ldx < K || ldy < N) return kAcross;
-  const int64_t col = ((d % ld) + ld) % ld;  // where y's rows start between two rows of x
-  if (col >= K * es && col + N * es <= ld) return kApart;
-  return d > -ld && d < ld && d + N * es <= ld && d >= K * es - ld ? kOwnRow : kAcross;
-}
-
 // Whether the plain row kernels (a wave per row, a thread per output) are
 // the faster ones: with few positions per tile and low ranks the matrix cores
 // multiply padding, and a round of 16-wave workgroups costs 7 us whatever its
@@ -362,14 +347,14 @@ int pl_wide_rows_launch(int32_t dtype, const void* x, int64_t ldx, int32_t K, vo
   if (rank_cap < 1 || rank_cap > kWideRankMax || tiles > (int64_t)1 << 24) return PL_WIDE_DECLINED;
   // y may lie over x: the workgroup of a tile reads all of its x rows before it
   // writes y, but several column ranges, or several tiles, run side by side
-  const int overlap = row_overlap(x, ldx, K, y, ldy, N, (int64_t)rows * row_len, pl_elem_size(dtype));
-  if (overlap == kAcross) return PL_WIDE_DECLINED;
+  const pl_overlap overlap = pl_row_overlap(x, ldx, K, y, ldy, N, (int64_t)rows * row_len, pl_elem_size(dtype));
+  if (overlap == pl_overlap::across) return PL_WIDE_DECLINED;
   const int step_cols = dtype == PL_F32 ? (int)pl_wide_shape<PL_F32>::kStepCols
                                         : (int)pl_wide_shape<PL_BF16>::kStepCols;
   // column ranges until the launch has about two workgroups per CU: each
   // range repeats the tile's shrink
   const int64_t steps = (N + step_cols - 1) / step_cols;
-  const int64_t want = overlap == kOwnRow ? 1 : std::max<int64_t>(1, 512 / std::max<int64_t>(1, tiles));
+  const int64_t want = overlap == pl_overlap::own_row ? 1 : std::max<int64_t>(1, 512 / std::max<int64_t>(1, tiles));
   const int64_t per = (steps + std::min(want, steps) - 1) / std::min(want, steps);
   pl_wide_args a;
   a.cols = (int32_t)(per * step_cols);

@@ -279,7 +279,7 @@ def lora_apply(
         if long_ok(plan, cache, x.shape[1], y.shape[1]) and not _host_paces_pair(plan, cache, x.shape[1], y.shape[1]):
             _long_launch(x, [y], cache, [module_name], plan, epilogue, _stream(x.device))
             return y
-        if _one_launch_ok(plan, cache, x.shape[1], y.shape[1]) and _own_rows(x, y):
+        if _one_launch_ok(plan, cache, x.shape[1], y.shape[1]):
             _decode_launch(x, [y], cache, [module_name], plan, None, epilogue, _stream(x.device))
             return y
     dt = _native.dtype_code(x.dtype)
@@ -577,10 +577,11 @@ def long_ok(plan: SgmvPlan, cache, in_features: int, out_features: int, modules:
     es = cache.dtype.itemsize
     if rank > FUSED_MAX_RANK:
         return es == 2 and rank <= LONG_MAX_RANK and tokens >= LONG_MIN_TOKENS
-    if in_features > FUSED_MAX_K or not _long_grid_fits(tokens, es, rank, out_features, modules):
+    if in_features > FUSED_MAX_K:
         return False
     pays = _long_pays_to_rank_32 if rank <= 32 else _long_pays_above_rank_32
-    return pays(tokens, es, rank, in_features, out_features, modules)
+    return (pays(tokens, es, rank, in_features, out_features, modules)
+            and _long_grid_fits(tokens, es, rank, out_features, modules))
 
 
 def _long_pays_to_rank_32(tokens: int, es: int, rank: int, K: int, N: int, modules: int) -> bool:
@@ -716,7 +717,7 @@ def _fused_launch(x, y, cache, module_name: str, plan: SgmvPlan, epilogue: int, 
     """pl_lora_fused on operands the caller has checked, or the two-launch path where long_ok prefers it."""
     K, N = x.shape[1], y.shape[1]
     if slices is None:
-        if _use_long(x, plan, cache, (N,), stream)[0]:
+        if long_ok(plan, cache, K, N) and stream == _stream(x.device):
             _long_launch(x, [y], cache, [module_name], plan, epilogue, stream)
             return
         slices = choose_slices(plan, N)
@@ -999,21 +1000,6 @@ def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -
     return (cache.decode_handoff and plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
             and plan.tokens_cap < _ONE_LAUNCH_MAX_TOKENS
             and (plan.tokens_cap < 256 or out_features <= 2 * in_features))
-
-
-def _own_rows(x: torch.Tensor, y: torch.Tensor) -> bool:
-    """Whether no row of y lies over another row of x.  The one launch writes the rows of a group of tokens while it
-    still reads those of others; the split pair reads all of x first."""
-    xs, ys = x.stride(0), y.stride(0)
-    (rows, K), N = x.shape, y.shape[1]
-    d = (y.data_ptr() - x.data_ptr()) // x.element_size()
-    if d >= (rows - 1) * xs + K or -d >= (rows - 1) * ys + N or rows == 1:
-        return True
-    if xs != ys:
-        return False
-    if K <= d % xs <= xs - N:  # between x's rows
-        return True
-    return -xs < d < xs and K - xs <= d <= xs - N
 
 
 def _decode_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, k_splits, epilogue: int, stream: int) -> None:

@@ -326,25 +326,32 @@ def test_graphs_captured_on_one_stream_replay_in_any_order(gpu, monkeypatch):
     assert len(captures) == 4 and len(set(captures)) == 2  # in each: for one module, then for two
 
 
-@pytest.mark.parametrize("kind,one", [("same", True), ("beside", True), ("next row", False), ("other stride", False)])
-def test_lora_apply_reads_x_before_an_overlapping_y(gpu, monkeypatch, kind, one):
-    """x and y in one buffer give what separate buffers give, bit for bit: in one launch where a row of y lies over its
-    own row of x at most, else by the split pair."""
-    launches = []
-    launch = sgmv._decode_launch
-    monkeypatch.setattr(sgmv, "_decode_launch", lambda *a: (launches.append(1), launch(*a))[1])
+@pytest.mark.parametrize("kind", ["same", "beside", "tail", "next row", "other stride"])
+@pytest.mark.parametrize("modules", [1, 2])
+def test_decode_launch_reads_x_before_an_overlapping_y(gpu, kind, modules):
+    """x and y in one buffer give what separate buffers give, bit for bit, in lora_apply and lora_decode_stacked: y is
+    x, beside it in packed rows, over its last columns, one row further, or of another row stride."""
+    print("case:", kind, modules, flush=True)
     g = torch.Generator().manual_seed(81)
-    T, K = 100, 1024
-    cache = make_cache({"a": {"m": peft_layer(g, K, K, 16, 32.0)}}, {"m": (K, K)}, 1, 16, gpu, torch.bfloat16)
+    T, K = 300, 1024
+    names = ["m", "n"][:modules]
+    cache = make_cache({"a": {m: peft_layer(g, K, K, 16, 32.0) for m in names}}, {m: (K, K) for m in names}, 1, 16, gpu,
+                       torch.bfloat16)
     plan = sgmv.SgmvPlan(cache.ensure_resident(["a"] * T), torch.ones(T, dtype=torch.int32, device=gpu), 1,
-                         cache.num_slots, distinct_slots=1)
+                         cache.num_slots, distinct_slots=1, group_tokens=16)
     buf = torch.randn(2 * T + 1, 2 * K, generator=g).bfloat16().to(gpu)
     x = buf[:T, :K]
-    y = {"same": x, "beside": buf[:T, K:], "next row": buf[1 : T + 1, :K],
-         "other stride": buf.view(-1, K)[: T]}[kind]
-    splits = sgmv.choose_k_splits(plan.group_cap, K, torch.bfloat16)
-    want = sgmv.lora_apply(x.clone(), y.clone(), cache, "m", plan, k_splits=splits)
-    assert not launches
-    sgmv.lora_apply(x, y, cache, "m", plan)
-    assert torch.equal(y, want) and bool(launches) == one
-    assert not sgmv.decode_waits_timed_out(gpu)
+    y = {"same": x, "beside": buf[:T, K:], "tail": buf[:T, K // 2 : K // 2 + K], "next row": buf[1 : T + 1, :K],
+         "other stride": buf.view(-1, K)[:T]}[kind]
+    other = torch.randn(T, K, generator=g).bfloat16().to(gpu)
+    want = [y.clone(), other.clone()][:modules]
+    apart = x.clone()
+    results = sgmv.lora_shrink_stacked(apart, cache, names, plan)
+    sgmv.lora_expand_stacked(results, want, cache, names)
+    ys = [y, other][:modules]
+    if modules == 1:
+        sgmv.lora_apply(x, y, cache, "m", plan)
+    else:
+        sgmv.lora_decode_stacked(x, ys, cache, names, plan)
+    assert all(torch.equal(a, b) for a, b in zip(ys, want))
+    _counters_clear(gpu)

@@ -759,27 +759,6 @@ def test_long_path_rule_stays_within_what_one_launch_can_hold(tokens, fout, modu
     assert sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.bfloat16), 4096, fout, modules) == want
 
 
-def test_rows_of_y_over_other_rows_of_x_are_seen():
-    """_own_rows against the addresses of the elements, for every offset and stride of two small matrices."""
-    from polylora_amd import sgmv
-
-    for xs in (3, 5, 8):
-        for ys in (3, 5, 8):
-            for K, N in ((3, 3), (2, 3), (3, 1), (1, 1)):
-                for off in range(30):
-                    buf = torch.zeros(60)
-                    for swap in (False, True):
-                        x = buf.as_strided((3, K), (xs, 1), off if swap else 10)
-                        y = buf.as_strided((3, N), (ys, 1), 10 if swap else off)
-                        cells = [[{t.storage_offset() + r * t.stride(0) + c for c in range(t.shape[1])} for r in range(3)]
-                                 for t in (x, y)]
-                        own = not any(cells[0][i] & cells[1][j] for i in range(3) for j in range(3) if i != j)
-                        # never taken for own rows when they are not; the exact answer for rows of one stride
-                        assert own or not sgmv._own_rows(x, y), (xs, ys, K, N, off, swap)
-                        if xs == ys:
-                            assert own == sgmv._own_rows(x, y), (xs, ys, K, N, off, swap)
-
-
 @pytest.mark.parametrize("groups,K,tokens,want", [
     (8, 4096, 1, 8), (16, 4096, 32, 8), (16, 4096, 33, 4), (16, 4096, 128, 4), (17, 4096, 8, 4), (16, 1024, 200, 4),
     (16, 8192, 1, 8), (16, 8192, 64, 8), (16, 3072, 8, 6), (16, 3072, 40, 4), (8, 11008, 8, 12), (8, 14336, 8, 16),
