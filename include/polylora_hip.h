@@ -166,8 +166,8 @@ int64_t pl_plan_group_capacity(int32_t rows, int32_t row_len, int32_t num_slots,
  *
  * Plan inputs of the kernels.  Every entry point below that takes tok,
  * groups and meta (pl_sgmv_shrink(_stacked), pl_sgmv_expand(_stacked),
- * pl_lora_apply, pl_lora_fused(_stacked), pl_lora_decode_stacked) reads
- * them as pl_plan_build or pl_plan_build_active wrote them: it walks the
+ * pl_lora_apply, pl_lora_fused(_stacked), pl_lora_long_stacked,
+ * pl_lora_decode_stacked) reads them as pl_plan_build or pl_plan_build_active wrote them: it walks the
  * group positions below meta[3] (records past the groups in use are empty)
  * and gives position p to XCD p % 8.  A plan built another way must follow
  * that format, meta[3] included: with meta[3] = 0 no group is read and the

@@ -8,8 +8,8 @@
 // read-modify-write wants (a probe over 705 MB of 28 KB rows: 5.7 TB/s with
 // 2 KB of each row per workgroup, 5.0 TB/s when a workgroup walks whole
 // rows).  Against one fused launch, whose workgroups run both phases, the
-// second launch costs about 5 us, and that is paid back from about 112 MB of
-// output traffic on, above rank 32 from 40 MB of x and y (sgmv.long_ok).  bf16, before -> after:
+// second launch costs about 5 us, and that is paid back by large and wide
+// outputs and by ranks above 32 (sgmv.long_ok).  bf16, before -> after:
 //   4096 -> 2 x 14336, rank 32, 24740 tokens  642 -> 564 us (5.4 TB/s in the expand)
 //   2048 -> 8192, rank 64, 4593 tokens         78 -> 46 us
 //   14336 -> 4096, rank 32, 24740 tokens      268 -> 230 us
