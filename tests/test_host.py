@@ -768,3 +768,14 @@ def test_k_splits_of_few_groups(groups, K, tokens, want):
     from polylora_amd import sgmv
 
     assert sgmv.choose_k_splits(groups, K, torch.bfloat16, tokens) == want
+
+
+@pytest.mark.parametrize("K,tokens,groups,want", [
+    (14336, 128, 24, False), (14336, 63, 24, True), (14336, 900, 97, True), (8192, 256, 80, False), (8184, 256, 24, True)])
+def test_lora_apply_over_a_long_k_takes_one_launch_for_few_tokens_or_many_groups(K, tokens, groups, want):
+    from types import SimpleNamespace as Obj
+
+    from polylora_amd import sgmv
+
+    plan = Obj(group_tokens=16, tokens_cap=tokens, group_cap=groups)
+    assert sgmv._one_launch_ok(plan, Obj(rank8_cap=64, decode_handoff=True), K, 4096) == want
