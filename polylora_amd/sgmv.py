@@ -185,9 +185,10 @@ def _workspace(device: torch.device, stream: int, position: int = 0) -> _Workspa
 # at most 16 groups: splits of 512 up to 8 while every expand workgroup sums
 # the planes of few rows (rank 64: K = 4096, 8 rows 8.9 -> 8.1, gate/up, 24 rows
 # 11.8 -> 10.6; rank 16, gate/up, 48 rows 9.8 -> 12.9, so only to 32 rows), and
-# above K = 8192 one per 896, up to 16 (8 rows, rank 64: K = 14336 12.2 -> 11.5,
-# K = 11008 11.1 -> 10.6; K = 8192 with 16 is slower, 8192 -> 28672, rank 16, 12
-# rows 10.3 -> 13.4, q/k/v 9.2 -> 10.1).
+# above K = 8192 one per 512, up to 16, where no module of that input is wider
+# than half of it (rank 64, 8 rows: 14336 -> 4096 12.2 -> 11.6, 11008 -> 4096 11.1
+# -> 10.4; K = 8192 with 16 is slower, 8192 -> 28672, rank 16, 12 rows 10.3 ->
+# 13.4, q/k/v 9.2 -> 10.1; 9984 -> 11712 and two more, 44 rows, 10.8 -> 14.2).
 _K_PER_SPLIT = 1024
 _TARGET_SHRINK_BLOCKS = 2048
 _MAX_K_SPLITS = 8
@@ -196,13 +197,14 @@ _FEWEST_GROUPS = 16
 _FEW_TOKENS = 32
 
 
-def choose_k_splits(group_cap: int, K: int, dtype: torch.dtype, tokens: int = 1) -> int:
-    """K splits of the shrink: about one per 1024 of K (at most 8), more for few groups (and few `tokens`), fewer when
-    the group count alone fills the GPU."""
+def choose_k_splits(group_cap: int, K: int, dtype: torch.dtype, tokens: int = 1, widest: int = 0) -> int:
+    """K splits of the shrink: about one per 1024 of K (at most 8), more for few groups (with few `tokens`, or a long K
+    whose `widest` output is narrow), fewer when the group count alone fills the GPU."""
     by_k = min(_MAX_K_SPLITS, max(1, -(-K // _K_PER_SPLIT)))
     if group_cap <= _FEWEST_GROUPS:
         if K > _MAX_K_SPLITS * _K_PER_SPLIT:
-            by_k = max(by_k, min(2 * _MAX_K_SPLITS, K // 896))
+            if 2 * widest <= K:
+                by_k = max(by_k, min(2 * _MAX_K_SPLITS, K // 512))
         elif tokens <= _FEW_TOKENS:
             by_k = max(by_k, min(_MAX_K_SPLITS, K // 512))
     if group_cap <= _FEW_GROUPS:
@@ -287,7 +289,7 @@ def lora_apply(
     arena, table, n_mod, column, ldt = _cache_args(cache, module_name)
     stream = _stream(x.device)
     rows = max(1, plan.tokens_cap)
-    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, x.dtype, plan, rows, ldt, k_splits)
+    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, x.dtype, plan, rows, ldt, k_splits, cache)
     ws = _workspace(x.device, stream)
     buf = ws.get(nbytes)
     ws.owner = None  # planes of an earlier separate shrink on this workspace are gone
@@ -359,17 +361,30 @@ def tiled_shapes_ok(x: torch.Tensor, out_features: int) -> bool:
 _GEOMETRY: dict[tuple, tuple[int, int, int]] = {}
 
 
+def _widest_output(cache, in_features: int) -> int:
+    """The widest output of the cache's modules of this input width, found once per cache and width: the same for a
+    module alone and with its siblings, which must split K alike to give the same bits."""
+    memo = cache.__dict__.setdefault("_widest_outputs", {})
+    got = memo.get(in_features)
+    if got is None:
+        got = memo[in_features] = max((s.out_features for s in cache.module_specs.values() if s.in_features == in_features),
+                                      default=0)
+    return got
+
+
 def _shrink_geometry(lib, dt: int, K: int, dtype: torch.dtype, plan: SgmvPlan, rows: int, ldt: int,
-                     k_splits: int | None) -> tuple[int, int, int]:
+                     k_splits: int | None, cache=None) -> tuple[int, int, int]:
     """(k_splits, planes, workspace bytes) of a shrink, computed once per shape."""
-    key = (dt, K, plan.group_cap, plan.group_tokens, rows, ldt, k_splits)
+    # a K of 8192 or less splits alike for any outputs
+    widest = _widest_output(cache, K) if K > _MAX_K_SPLITS * _K_PER_SPLIT and cache is not None else 0
+    key = (dt, K, plan.group_cap, plan.group_tokens, rows, ldt, k_splits, widest)
     geo = _GEOMETRY.get(key)
     if geo is None:
         if k_splits is None:
             # the extra splits of few groups do not pay for their planes above rank 64 (37 rows, 14336 -> 4096, rank
             # 128: 16 splits 15.1 to 16.0 us, 8 splits 15.0)
             cap = plan.group_cap if ldt <= FUSED_MAX_RANK else max(plan.group_cap, _FEW_GROUPS + 1)
-            splits = choose_k_splits(cap, K, dtype, rows)
+            splits = choose_k_splits(cap, K, dtype, rows, widest)
         else:
             splits = k_splits
         planes = int(lib.pl_shrink_planes(dt, K, splits, plan.group_tokens))
@@ -445,7 +460,7 @@ def lora_shrink_stacked(x: torch.Tensor, cache, module_names: list, plan: SgmvPl
     if stream is None:
         stream = _stream(x.device)
     rows = max(1, plan.tokens_cap)
-    splits, planes, nbytes = _shrink_geometry(lib, dt, K, x.dtype, plan, rows, ldt, k_splits)
+    splits, planes, nbytes = _shrink_geometry(lib, dt, K, x.dtype, plan, rows, ldt, k_splits, cache)
     wss, bufs, ptrs, size = _workspace_set(x.device, stream, n, nbytes)
     arena, table, n_mod, _, _ = _cache_args(cache, module_names[0])
     rc = _native.calls().pl_sgmv_shrink_stacked(
@@ -1015,7 +1030,7 @@ def _decode_launch(x, ys: list, cache, module_names: list, plan: SgmvPlan, k_spl
     dt = _native.dtype_code(dtype)
     ldt = -(-cache.rank8_cap // 32) * 32  # plane rows of whole 128-byte lines
     rows = max(1, plan.tokens_cap)
-    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, dtype, plan, rows, ldt, k_splits)
+    splits, _, nbytes = _shrink_geometry(_native.load(), dt, K, dtype, plan, rows, ldt, k_splits, cache)
     wss, _, ptrs, size = _workspace_set(device, stream, n, nbytes)
     for ws in wss:
         ws.owner = None  # any earlier shrink's planes there are overwritten by this launch

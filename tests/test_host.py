@@ -759,15 +759,26 @@ def test_long_path_rule_stays_within_what_one_launch_can_hold(tokens, fout, modu
     assert sgmv.long_ok(plan, Obj(rank8_cap=rank, dtype=torch.bfloat16), 4096, fout, modules) == want
 
 
-@pytest.mark.parametrize("groups,K,tokens,want", [
-    (8, 4096, 1, 8), (16, 4096, 32, 8), (16, 4096, 33, 4), (16, 4096, 128, 4), (17, 4096, 8, 4), (16, 1024, 200, 4),
-    (16, 8192, 1, 8), (16, 8192, 64, 8), (16, 3072, 8, 6), (16, 3072, 40, 4), (8, 11008, 8, 12), (8, 14336, 8, 16),
-    (16, 14336, 128, 16), (17, 14336, 8, 8), (128, 2048, 256, 4), (129, 2048, 256, 2)])
-def test_k_splits_of_few_groups(groups, K, tokens, want):
-    """More splits only where their planes are summed for few rows or the K chain is the longest."""
+@pytest.mark.parametrize("groups,K,tokens,widest,want", [
+    (8, 4096, 1, 14336, 8), (16, 4096, 32, 14336, 8), (16, 4096, 33, 1024, 4), (16, 4096, 128, 4096, 4),
+    (17, 4096, 8, 4096, 4), (16, 1024, 200, 1024, 4), (16, 8192, 1, 1024, 8), (16, 8192, 64, 28672, 8),
+    (16, 3072, 8, 3072, 6), (16, 3072, 40, 3072, 4), (8, 11008, 8, 4096, 16), (8, 14336, 8, 4096, 16),
+    (16, 14336, 128, 7168, 16), (16, 14336, 8, 7176, 8), (8, 9984, 44, 11712, 8), (17, 14336, 8, 4096, 8),
+    (128, 2048, 256, 2048, 4), (129, 2048, 256, 2048, 2)])
+def test_k_splits_of_few_groups(groups, K, tokens, widest, want):
+    """More splits only where their planes are summed for few rows, or for narrow outputs of the longest K."""
+    from types import SimpleNamespace as Obj
+
     from polylora_amd import sgmv
 
-    assert sgmv.choose_k_splits(groups, K, torch.bfloat16, tokens) == want
+    assert sgmv.choose_k_splits(groups, K, torch.bfloat16, tokens, widest) == want
+    # as the launches ask for it: by the widest of the modules that share the input width, whichever they serve
+    specs = {"a": Obj(in_features=K, out_features=8), "b": Obj(in_features=K, out_features=widest),
+             "c": Obj(in_features=K + 8, out_features=1 << 20)}
+    lib = Obj(pl_shrink_planes=lambda *a: a[2], pl_shrink_workspace_bytes=lambda *a: 0)
+    plan = Obj(group_cap=groups, group_tokens=16)
+    cache = Obj(module_specs=specs)
+    assert sgmv._shrink_geometry(lib, 7, K, torch.bfloat16, plan, tokens, 64, None, cache)[0] == want
 
 
 @pytest.mark.parametrize("K,tokens,groups,want", [
