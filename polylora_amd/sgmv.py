@@ -1005,10 +1005,12 @@ def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -
     128: 13.8 -> 15.4 us), and for many rows of wide outputs (256 rows, 4096 ->
     14336, rank 64: 18.6 -> 19.5 us).  With a long K the expand workgroups of
     few groups hold their places on the GPU for the whole of the shrink, so
-    from K = 8192 on the pair is the faster one from 64 tokens on in up to 80
-    group positions (14336 -> 4096, 8 adapters, rank 64, 128 tokens 11.2 ->
-    12.4 us; 12288 -> 12288, 2 adapters, rank 16, 128 tokens 9.5 -> 12.1; 900
-    tokens of 40 adapters 26.4 -> 23.2).  Measured, and taken, up to the tokens
+    from K = 8192 on and 2048 outputs the pair is the faster one for half a
+    million outputs of up to 80 group positions (14336 -> 4096, 8 adapters, rank
+    64, 128 tokens 11.2 -> 12.4 us; 12288 -> 12288, 2 adapters, rank 16, 128
+    tokens 9.5 -> 12.1; less, or 1024 outputs, the host paces: 14336 -> 1024, 4
+    adapters, 320 tokens, calls back to back 10.8 -> 10.1; 14336 -> 4096, 40
+    adapters, 900 tokens 26.4 -> 23.2).  Measured, and taken, up to the tokens
     from which plans have 64-token groups (on the GPU, 150 adapters of rank
     64: 4096 -> 4096, 2047 tokens 34.6 -> 33.4 us, 8191 tokens 84.0 -> 83.6;
     14336 -> 4096, 4095 tokens 104 -> 97; 1024 -> 1024, 8191 tokens 28.1 ->
@@ -1019,7 +1021,8 @@ def _one_launch_ok(plan: SgmvPlan, cache, in_features: int, out_features: int) -
     """
     return (cache.decode_handoff and plan.group_tokens == _native.PL_GROUP_TOKENS_SHORT and cache.rank8_cap <= 64
             and plan.tokens_cap < _ONE_LAUNCH_MAX_TOKENS
-            and (in_features < 8192 or plan.tokens_cap < 64 or plan.group_cap > 80)
+            and (in_features < 8192 or out_features < 2048 or plan.tokens_cap * out_features < 1 << 19
+                 or plan.group_cap > 80)
             and (plan.tokens_cap < 256 or out_features <= 2 * in_features))
 
 

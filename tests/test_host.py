@@ -781,12 +781,13 @@ def test_k_splits_of_few_groups(groups, K, tokens, widest, want):
     assert sgmv._shrink_geometry(lib, 7, K, torch.bfloat16, plan, tokens, 64, None, cache)[0] == want
 
 
-@pytest.mark.parametrize("K,tokens,groups,want", [
-    (14336, 128, 24, False), (14336, 63, 24, True), (14336, 900, 97, True), (8192, 256, 80, False), (8184, 256, 24, True)])
-def test_lora_apply_over_a_long_k_takes_one_launch_for_few_tokens_or_many_groups(K, tokens, groups, want):
+@pytest.mark.parametrize("K,N,tokens,groups,want", [
+    (14336, 4096, 128, 24, False), (14336, 4096, 127, 24, True), (14336, 4096, 900, 97, True),
+    (8192, 8192, 256, 80, False), (8184, 8192, 256, 24, True), (14336, 2040, 600, 48, True), (12288, 12288, 48, 8, False)])
+def test_lora_apply_over_a_long_k_takes_one_launch_for_few_outputs_or_many_groups(K, N, tokens, groups, want):
     from types import SimpleNamespace as Obj
 
     from polylora_amd import sgmv
 
     plan = Obj(group_tokens=16, tokens_cap=tokens, group_cap=groups)
-    assert sgmv._one_launch_ok(plan, Obj(rank8_cap=64, decode_handoff=True), K, 4096) == want
+    assert sgmv._one_launch_ok(plan, Obj(rank8_cap=64, decode_handoff=True), K, N) == want
